@@ -102,6 +102,30 @@ def test_mlp_grad_vs_oracle(torch_mod, n):
         assert np.linalg.norm(g[lo:hi] - gref[lo:hi]) <= 1e-2 * np.linalg.norm(gref[lo:hi]) + 1e-9
 
 
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 129, 128 * 1024 + 5])
+def test_mlp_grad_ragged_batches(torch_mod, n):
+    """Part-filled chains, waves and workgroups, and more than one pass of a
+    workgroup. The sums are in FP32 (relative 1e-5 at these depths); an
+    activation or operand near a rounding boundary may round to the other
+    neighbour in BF16, 2^-8 of it, which is the bound for one sample."""
+    torch = torch_mod
+    from pyshocks_amd.learned import Trainer
+
+    rng = np.random.default_rng(20 + n)
+    p = _params(11, 0.3)
+    rec = np.zeros((n, M.RECORD), dtype=np.float32)
+    rec[:, :5] = M.features(rng.standard_normal((n, 5)))
+    rec[:, 5:8] = rng.standard_normal((n, 3)) * 0.1
+    rec[:, 8:11] = rng.dirichlet(np.ones(3), n)
+    rec[:, 11] = rng.uniform(0.1, 1.0, n)
+    tr = Trainer(_weights(torch, p), lambda_js=0.05, delta=1e-3)
+    g = tr.loss_and_grad(torch.tensor(rec, device="cuda")).cpu().numpy().astype(np.float64)
+    loss, gref = M.loss_and_grad(p, rec, lambda_js=0.05, delta=1e-3)
+    tol = 2.0**-8 if n < 64 else 2e-3
+    assert abs(g[-1] - loss) <= tol * abs(loss)
+    assert np.linalg.norm(g[:-1] - gref) <= tol * np.linalg.norm(gref)
+
+
 def test_training_reduces_loss(torch_mod):
     """The device training loop fits weights that pick the best candidate
     of synthetic records."""
