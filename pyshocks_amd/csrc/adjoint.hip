@@ -43,110 +43,196 @@
 namespace psa {
 namespace {
 
-constexpr int kVjpBlock = 256;              // computing cells per workgroup
-constexpr int kVjpThreads = 2 * kVjpBlock;  // split form: a thread per cell and side
+constexpr int kVjpBlock = 256;          // threads and computing cells per workgroup
+constexpr int kVjpWaves = kVjpBlock / 64;
 constexpr int kVjpOut = kVjpBlock - 6;  // output cells per workgroup
 
-// cell gm of a periodic array with n interior cells and g ghosts
-template <typename T>
-__device__ __forceinline__ T load_periodic(const T *__restrict__ u, int64_t gm,
-                                           int64_t n, int g) {
-  int64_t k = (gm - g) % n;
-  if (k < 0) k += n;
-  return u[g + k];
-}
+// The cells first, first + 1, .. of a periodic array with n interior cells and
+// g ghosts, first >= g - n (in [g - n, g + n) but for the tiniest grids). A
+// subtraction for each index instead of a 64-bit remainder, which cost as
+// much as a reverse stage.
+struct PeriodicSpan {
+  int64_t lo;  // the first cell's interior index, in [0, n)
+  int64_t n;
+  int g;
 
-// 1 / x for a positive normal FP64 x: the hardware reciprocal refined by
-// two Newton steps.
-__device__ __forceinline__ double rcp_refined(double x) {
-  double inv = __builtin_amdgcn_rcp(x);
-  double e = fma(-x, inv, 1.0);
-  inv = fma(inv, e, inv);
-  e = fma(-x, inv, 1.0);
-  return fma(inv, e, inv);
-}
-
-// The normalised WENO-JS weights w_k of a_k = d_k / e_k^2 and the
-// reciprocals ie_k = 1 / e_k of the indicators e_k = eps + beta_k. FP64: one
-// refined reciprocal of e0 e1 e2 and one of the sum of the a_k when both are
-// positive normal numbers (6 divisions fewer per side, a few ulps from
-// them), else the divisions; FP32: the divisions.
-template <typename T>
-__device__ __forceinline__ void weno_weights_inv(T e0, T e1, T e2, T &w0, T &w1, T &w2,
-                                                 T &ie0, T &ie1, T &ie2) {
-  using C = Weno5Coeffs<T>;
-  if constexpr (std::is_same<T, double>::value) {
-    const double e01 = e0 * e1;
-    const double den = e01 * e2;
-    if (__builtin_amdgcn_class(den, 0x100)) {
-      const double inv = rcp_refined(den);
-      ie0 = (e1 * e2) * inv;
-      ie1 = (e0 * e2) * inv;
-      ie2 = e01 * inv;
-      const double a0 = C::d0 * (ie0 * ie0);
-      const double a1 = C::d1 * (ie1 * ie1);
-      const double a2 = C::d2 * (ie2 * ie2);
-      const double s = (a0 + a1) + a2;
-      if (__builtin_amdgcn_class(s, 0x100)) {
-        const double is = rcp_refined(s);
-        w0 = a0 * is;
-        w1 = a1 * is;
-        w2 = a2 * is;
-        return;
-      }
+  __device__ __forceinline__ PeriodicSpan(int64_t first, int64_t n_, int g_)
+      : n(n_), g(g_) {
+    int64_t k = first - g_;
+    if (k < 0) {
+      k += n;
+      if (k < 0) k = k % n + n;
     }
+    if (k >= n) k %= n;
+    lo = k;
   }
-  const T a0 = C::d0 / (e0 * e0);
-  const T a1 = C::d1 / (e1 * e1);
-  const T a2 = C::d2 / (e2 * e2);
-  const T s = (a0 + a1) + a2;
-  w0 = a0 / s;
-  w1 = a1 / s;
-  w2 = a2 / s;
-  ie0 = T(1) / e0;
-  ie1 = T(1) / e1;
-  ie2 = T(1) / e2;
+  template <typename T>
+  __device__ __forceinline__ T load(const T *__restrict__ u, int j) const {
+    int64_t k = lo + j;
+    if (k >= n) {
+      k -= n;
+      if (k >= n) k %= n;
+    }
+    return u[g + k];
+  }
+};
+
+// 1 / x for a positive normal FP64 x: the hardware reciprocal y (relative
+// error e below 1e-7) with e + e^2 added, which leaves e^3.
+__device__ __forceinline__ double rcp_refined(double x) {
+  const double y = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, y, 1.0);
+  return fma(y, fma(e, e, e), y);
 }
 
-// Right reconstruction (value at x_{i+1/2}) of a cell from
-// (u[i-2], ..., u[i+2]) and its gradient with respect to those five values.
+// Both reconstructions of a cell and what their gradients take. The forward
+// kernels' difference form: D_k the first differences of the stencil, s_k the
+// second ones, t = (2 D1 + s0, D1 + D2, s2 - 2 D2), e_k = 4 (eps + beta_k) =
+// 4 eps + 13/3 s_k^2 + t_k^2, T0 = s1 - s0, T1 = s2 - s1;
+//   ur = u + (D1 + 2 D2) / 6 - mR,  mR = wR0 T0 / 3 + wR2 T1 / 6,
+//   ul = u - (2 D1 + D2) / 6 + mL,  mL = wL2 T1 / 3 + wL0 T0 / 6,
+// the weights indexed by their indicator: wR_k ~ (1, 6, 3) / e_k^2, wL_k ~
+// (3, 6, 1) / e_k^2, normalised. With
+//   dur/de_k = -2 zR_k,  zR_k = wR_k (hR_k - ur) / e_k   (left alike)
+// the two sides share everything up to the weights, and their contributions
+// meet in one set of derivatives of e_k (weno_cell_scatter).
 template <typename T>
-__device__ __forceinline__ T weno_side_grad(T um2, T um1, T u0, T up1, T up2,
-                                            T eps, T G[5]) {
+struct CellStates {
+  T s[3], t[3];
+  T qR[3], qL[3];  // w_k (h_k - value) of the right and left state
+  T ie[3];         // 1 / e_k
+  T wR0, wR2, wL0, wL2;
+};
+
+// The weights of both sides and 1 / e_k. FP64: one refined reciprocal of
+// e0 e1 e2 and one of the product of the two weight sums where both are
+// positive normal numbers, else the divisions; FP32: the divisions.
+template <typename T>
+__device__ __forceinline__ void weno_cell_weights(T e0, T e1, T e2, T ie[3], T wR[3],
+                                                  T wL[3]) {
+  bool fast = false;
+  if constexpr (std::is_same<T, double>::value) {
+    const double e01 = e0 * e1, e12 = e1 * e2, e02 = e0 * e2;
+    const double den = e01 * e2;
+    const double inv = rcp_refined(den);
+    ie[0] = e12 * inv;
+    ie[1] = e02 * inv;
+    ie[2] = e01 * inv;
+    const double x0 = ie[0] * ie[0], x1 = 6.0 * (ie[1] * ie[1]), x2 = ie[2] * ie[2];
+    const double aR = fma(3.0, x2, x0 + x1), aL = fma(3.0, x0, x2 + x1);
+    const double aa = aR * aL;
+    const double ia = rcp_refined(aa);
+    const double iR = aL * ia, iL = aR * ia;
+    wR[0] = x0 * iR;
+    wR[1] = x1 * iR;
+    wR[2] = 3.0 * (x2 * iR);
+    wL[0] = 3.0 * (x0 * iL);
+    wL[1] = x1 * iL;
+    wL[2] = x2 * iL;
+    fast = __builtin_amdgcn_class(den, 0x100) && __builtin_amdgcn_class(aa, 0x100);
+  }
+  if (__builtin_expect(!fast, std::is_same<T, float>::value)) {
+    using C = Weno5Coeffs<T>;
+    const T q0 = e0 * e0, q1 = e1 * e1, q2 = e2 * e2;
+    const T a0 = C::d0 / q0, a1 = C::d1 / q1, a2 = C::d2 / q2;
+    const T l0 = C::d2 / q0, l2 = C::d0 / q2;
+    const T aR = (a0 + a1) + a2, aL = (l2 + a1) + l0;
+    wR[0] = a0 / aR;
+    wR[1] = a1 / aR;
+    wR[2] = a2 / aR;
+    wL[0] = l0 / aL;
+    wL[1] = a1 / aL;
+    wL[2] = l2 / aL;
+    ie[0] = T(1) / e0;
+    ie[1] = T(1) / e1;
+    ie[2] = T(1) / e2;
+  }
+}
+
+// The differences of the stencil (into c.s, c.t) and the indicators e_k.
+template <typename T>
+__device__ __forceinline__ void weno_cell_indicators(const T v[5], T eps4, T &D1, T &D2,
+                                                     CellStates<T> &c, T e[3]) {
   using C = Weno5Coeffs<T>;
-  const T t00 = (u0 - T(2) * um1) + um2;
-  const T t01 = (T(3) * u0 - T(4) * um1) + um2;
-  const T t10 = (up1 - T(2) * u0) + um1;
-  const T t11 = up1 - um1;
-  const T t20 = (up2 - T(2) * up1) + u0;
-  const T t21 = (up2 - T(4) * up1) + T(3) * u0;
-  const T b0 = C::a0 * (t00 * t00) + C::a1 * (t01 * t01);
-  const T b1 = C::a0 * (t10 * t10) + C::a1 * (t11 * t11);
-  const T b2 = C::a0 * (t20 * t20) + C::a1 * (t21 * t21);
-  T h0, h1, h2;
-  weno_uhat(um2, um1, u0, up1, up2, h0, h1, h2);
+  const T D0 = v[1] - v[0];
+  D1 = v[2] - v[1];
+  D2 = v[3] - v[2];
+  const T D3 = v[4] - v[3];
+  c.s[0] = D1 - D0;
+  c.s[1] = D2 - D1;
+  c.s[2] = D3 - D2;
+  c.t[0] = fma(T(2), D1, c.s[0]);
+  c.t[1] = D2 + D1;
+  c.t[2] = fma(T(-2), D2, c.s[2]);
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    e[k] = fma(c.t[k], c.t[k], fma(C::a0x4, c.s[k] * c.s[k], eps4));
+}
 
-  const T e0 = eps + b0, e1 = eps + b1, e2 = eps + b2;
-  T w0, w1, w2, ie0, ie1, ie2;
-  weno_weights_inv(e0, e1, e2, w0, w1, w2, ie0, ie1, ie2);
-  const T r = (w0 * h0 + w1 * h1) + w2 * h2;
+// Both states from the middle candidates and the weights c.wR0 .. c.wL2.
+template <typename T>
+__device__ __forceinline__ void weno_cell_values(T u, T D1, T D2, const CellStates<T> &c,
+                                                 T &mR, T &mL, T &ul, T &ur) {
+  const T a = (c.s[1] - c.s[0]) * T(1.0 / 6.0), b = (c.s[2] - c.s[1]) * T(1.0 / 6.0);
+  mR = fma(c.wR0, a + a, c.wR2 * b);
+  mL = fma(c.wL2, b + b, c.wL0 * a);
+  ur = fma(c.t[1] + D2, T(1.0 / 6.0), u) - mR;
+  ul = fma(c.t[1] + D1, T(-1.0 / 6.0), u) + mL;
+}
 
-  // dr/dbeta_k = -2 omega_k (uhat_k - r) / (eps + beta_k)
-  const T q0 = T(-2) * w0 * (h0 - r) * ie0;
-  const T q1 = T(-2) * w1 * (h1 - r) * ie1;
-  const T q2 = T(-2) * w2 * (h2 - r) * ie2;
-  // dr/dt_kj = dr/dbeta_k * 2 a_j t_kj
-  const T p00 = q0 * (T(2) * C::a0) * t00, p01 = q0 * (T(2) * C::a1) * t01;
-  const T p10 = q1 * (T(2) * C::a0) * t10, p11 = q1 * (T(2) * C::a1) * t11;
-  const T p20 = q2 * (T(2) * C::a0) * t20, p21 = q2 * (T(2) * C::a1) * t21;
+// WENO-JS states of a cell from its stencil and what the gradient takes.
+template <typename T>
+__device__ __forceinline__ void weno_cell_states(const T v[5], T eps4, CellStates<T> &c,
+                                                 T &ul, T &ur) {
+  T D1, D2, e[3], wR[3], wL[3];
+  weno_cell_indicators(v, eps4, D1, D2, c, e);
+  weno_cell_weights(e[0], e[1], e[2], c.ie, wR, wL);
+  c.wR0 = wR[0];
+  c.wR2 = wR[2];
+  c.wL0 = wL[0];
+  c.wL2 = wL[2];
+  T mR, mL;
+  weno_cell_values(v[2], D1, D2, c, mR, mL, ul, ur);
+  // hR_k - ur = (mR - T0/3, mR, mR - T1/6), hL_k - ul = (T0/6 - mL, -mL, T1/3 - mL)
+  const T a = (c.s[1] - c.s[0]) * T(1.0 / 6.0), b = (c.s[2] - c.s[1]) * T(1.0 / 6.0);
+  c.qR[0] = wR[0] * (mR - (a + a));
+  c.qR[1] = wR[1] * mR;
+  c.qR[2] = wR[2] * (mR - b);
+  c.qL[0] = wL[0] * (a - mL);
+  c.qL[1] = -(wL[1] * mL);
+  c.qL[2] = wL[2] * ((b + b) - mL);
+}
 
-  G[0] = (p00 + p01) + w0 * C::c2;
-  G[1] = (T(-2) * p00 - T(4) * p01 + p10 - p11) - w0 * C::c7 - w1 * C::c1;
-  G[2] = (p00 + T(3) * p01 - T(2) * p10 + p20 + T(3) * p21) + w0 * C::c11 +
-         w1 * C::c5 + w2 * C::c2;
-  G[3] = (p10 + p11 - T(2) * p20 - T(4) * p21) + w1 * C::c2 + w2 * C::c5;
-  G[4] = (p20 + p21) - w2 * C::c1;
-  return r;
+// cR dur/dv + cL dul/dv of a cell: through the weights (z_k = (cR qR_k +
+// cL qL_k) / e_k, de_k = 26/3 s_k ds_k + 2 t_k dt_k; none with FIXED, weights
+// that do not depend on v), through T0 and T1 at fixed weights and through the
+// middle candidates, from the second to the first differences and to v.
+template <typename T>
+__device__ __forceinline__ void weno_cell_scatter(const CellStates<T> &c, T cR, T cL,
+                                                  bool fixed, T P[5]) {
+  T at[3], as[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const T z = fixed ? T(0)
+                      : T(-4) * (fma(cR, c.qR[k], cL * c.qL[k]) * c.ie[k]);
+    at[k] = z * c.t[k];
+    as[k] = T(13.0 / 3.0) * (z * c.s[k]);
+  }
+  const T aT0 = fma(T(-2) * cR, c.wR0, cL * c.wL0) * T(1.0 / 6.0);
+  const T aT1 = fma(T(2) * cL, c.wL2, -(cR * c.wR2)) * T(1.0 / 6.0);
+  as[0] = (as[0] - aT0) + at[0];
+  as[1] = as[1] + (aT0 - aT1);
+  as[2] = (as[2] + aT1) + at[2];
+  const T h = (cR - cL) * T(1.0 / 6.0);
+  // cR/6 - cL/3 = h - cL/6, cR/3 - cL/6 = h + cR/6
+  const T g1 = (as[0] - as[1]) + (fma(T(2), at[0], at[1]) + fma(T(-1.0 / 6.0), cL, h));
+  const T g2 = (as[1] - as[2]) + (fma(T(-2), at[2], at[1]) + fma(T(1.0 / 6.0), cR, h));
+  // v_k: D_{k-1} + ... (D0 takes -as0, D3 takes as2)
+  P[0] = as[0];
+  P[1] = -as[0] - g1;
+  P[2] = (g1 - g2) + (cR + cL);
+  P[3] = g2 - as[2];
+  P[4] = as[2];
 }
 
 template <typename T>
@@ -169,52 +255,11 @@ struct VjpArgs {
   T eps;
   T vconst;
   const float *mlp;   // LEARNED: the network's parameters (PSA_MLP_NPARAM FP32)
-  T eps4;             // LEARNED: 4 eps (the fused indicators carry 4 beta)
+  T eps4;             // 4 eps (the indicators carry 4 beta)
   T tau;              // LEARNED: shock threshold
   T sigma;            // LEARNED: smooth threshold
   T alpha;            // Lax-Friedrichs: the global speed max|state| (in-kernel)
 };
-
-// Regime of a cell (mlp_regime) from its right stencil with the indicator
-// arithmetic of the forward kernels (reconstruct_cells: shared first and
-// second differences, 4 beta, one multiply-add each), so that the reverse
-// kernels see the regime the forward took.
-template <typename T>
-__device__ __forceinline__ int learned_regime5(T v0, T v1, T v2, T v3, T v4, T eps4,
-                                               T tau, T sigma) {
-  using C = Weno5Coeffs<T>;
-  const T D0 = v1 - v0, D1 = v2 - v1, D2 = v3 - v2, D3 = v4 - v3;
-  const T s0 = D1 - D0, s1 = D2 - D1, s2 = D3 - D2;
-  const T E0 = C::a0x4 * (s0 * s0), E1 = C::a0x4 * (s1 * s1), E2 = C::a0x4 * (s2 * s2);
-  const T t01 = fma(T(2), D1, s0);
-  const T t11 = D2 + D1;
-  const T t21 = fma(T(-2), D2, s2);
-  return mlp_regime(fma(t01, t01, E0), fma(t11, t11, E1), fma(t21, t21, E2), eps4, tau,
-                    sigma);
-}
-
-// Gradient of the candidates with respect to the stencil: G += sum_k c_k
-// d uhat_k / dv (weno.py:231-239 taps in the order of weno_side_grad).
-template <typename T>
-__device__ __forceinline__ void uhat_grad(T c0, T c1, T c2, T G[5]) {
-  using C = Weno5Coeffs<T>;
-  G[0] += c0 * C::c2;
-  G[1] += -(c0 * C::c7) - c1 * C::c1;
-  G[2] += (c0 * C::c11 + c1 * C::c5) + c2 * C::c2;
-  G[3] += c1 * C::c2 + c2 * C::c5;
-  G[4] += -(c2 * C::c1);
-}
-
-// Ideal-weight reconstruction (mlp_combine_ideal) and its stencil gradient.
-template <typename T>
-__device__ __forceinline__ T ideal_side_grad(T v0, T v1, T v2, T v3, T v4, T G[5]) {
-  T h0, h1, h2;
-  weno_uhat(v0, v1, v2, v3, v4, h0, h1, h2);
-#pragma unroll
-  for (int k = 0; k < 5; ++k) G[k] = T(0);
-  uhat_grad(T(0.1), T(1) - T(0.1) - T(0.3), T(0.3), G);
-  return mlp_combine_ideal(h0, h1, h2);
-}
 
 // A weight as the forward kernels' BF16 operand (round to nearest even, on
 // the bit pattern: the parameters are uniform, so this stays in scalar
@@ -244,210 +289,314 @@ __device__ __forceinline__ double mlp_weight<double>(const float *__restrict__ P
   return __hiloint2double(static_cast<int>(hi), 0);
 }
 
-// Network reconstruction of one side, r = h1 + w0 (h0 - h1) + w2 (h2 - h1)
-// with w = softmax(z) of the network on x = (v - mean) / max|v - mean|, and
-// its stencil gradient: the candidates' part with (w0, 1 - w0 - w2, w2), the
-// weights' part back through softmax, the three layers (ReLU masks of this
-// evaluation) and the normalisation. P: the parameters (weights rounded as
-// mlp_weight, b3 + ln d summed in FP32 as the forward's accumulator start).
-// Layer 2 runs row by row, so 32 values of T are live.
+// The network of the learned kernels in LDS, its weights as the forward
+// kernels round them (mlp_weight) and b3 + ln d summed in FP32 as the
+// forward's accumulator start, with room for one layer of the two sides that a
+// wave evaluates at once and the list of the workgroup's learned cells.
+template <typename T, bool USED>
+struct VjpNet {
+  int count;
+  unsigned short cell[kVjpBlock];
+  T w1[MLP_HID][MLP_IN], b1[MLP_HID];
+  T w2[MLP_HID][MLP_HID + 1], b2[MLP_HID];
+  T w3[MLP_OUT][MLP_HID], b3[MLP_OUT + 1];
+  __align__(16) T h[kVjpWaves][2][MLP_HID];
+};
 template <typename T>
-__device__ __forceinline__ T learned_side_grad(const float *__restrict__ P, T v0, T v1,
-                                               T v2, T v3, T v4, T G[5]) {
-  const T v[5] = {v0, v1, v2, v3, v4};
-  const T mean = (((v0 + v4) + (v1 + v3)) + v2) * T(0.2);
-  T d[5], x[5];
-  int km = 0;
+struct VjpNet<T, false> {};
+
+// Fills the network (a barrier must follow).
+template <typename T>
+__device__ __forceinline__ void vjp_net_load(VjpNet<T, true> &net,
+                                             const float *__restrict__ P) {
+  const int tid = threadIdx.x;
+  if (tid == 0) net.count = 0;
+  for (int i = tid; i < MLP_HID * MLP_HID; i += kVjpBlock)
+    net.w2[i / MLP_HID][i % MLP_HID] = mlp_weight<T>(P, MLP_W2 + i);
+  if (tid < MLP_HID * MLP_IN) net.w1[tid / MLP_IN][tid % MLP_IN] = mlp_weight<T>(P, MLP_W1 + tid);
+  if (tid < MLP_OUT * MLP_HID)
+    net.w3[tid / MLP_HID][tid % MLP_HID] = mlp_weight<T>(P, MLP_W3 + tid);
+  if (tid < MLP_HID) {
+    net.b1[tid] = static_cast<T>(P[MLP_B1 + tid]);
+    net.b2[tid] = static_cast<T>(P[MLP_B2 + tid]);
+  }
+  const float lnd[3] = {MLP_LN_D0, MLP_LN_D1, MLP_LN_D2};
+#pragma unroll
+  for (int o = 0; o < MLP_OUT; ++o)
+    if (tid == o) net.b3[o] = static_cast<T>(P[MLP_B3 + o] + lnd[o]);
+}
+
+// Sum over the 32 lanes of each half of the wave, to every lane of the half:
+// DPP moves within the rows of 16 lanes, a swizzle between the two rows.
+template <int CTRL>
+__device__ __forceinline__ float dpp_value(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_value(double v) {
+  return __hiloint2double(
+      __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, true),
+      __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float other_row(float v) {  // lane ^ 16
+  return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401F));
+}
+__device__ __forceinline__ double other_row(double v) {
+  return __hiloint2double(__builtin_amdgcn_ds_swizzle(__double2hiint(v), 0x401F),
+                          __builtin_amdgcn_ds_swizzle(__double2loint(v), 0x401F));
+}
+template <typename T>
+__device__ __forceinline__ T half_sum(T v) {
+  v += dpp_value<0xB1>(v);   // quad_perm [1, 0, 3, 2]
+  v += dpp_value<0x4E>(v);   // quad_perm [2, 3, 0, 1]
+  v += dpp_value<0x141>(v);  // row_half_mirror
+  v += dpp_value<0x140>(v);  // row_mirror
+  return v + other_row(v);
+}
+
+// The normalised inputs x = (v - mean) / s of the network, s = |d_km| =
+// max|d|, d = v - mean; inv = 1 / s (0 where s = 0), sg = sgn(d_km).
+template <typename T>
+__device__ __forceinline__ void learned_inputs(const T v[5], T x[5], T &inv, T &sg, int &km) {
+  const T mean = (((v[0] + v[4]) + (v[1] + v[3])) + v[2]) * T(0.2);
   T s = T(0);
+  sg = T(-1);
+  km = 0;
 #pragma unroll
   for (int k = 0; k < 5; ++k) {
-    d[k] = v[k] - mean;
-    if (fabs(d[k]) > s) {
-      s = fabs(d[k]);
+    x[k] = v[k] - mean;
+    if (fabs(x[k]) > s) {
+      s = fabs(x[k]);
+      sg = x[k] > T(0) ? T(1) : T(-1);
       km = k;
     }
   }
-  const T inv = s > T(0) ? T(1) / s : T(0);
+  inv = s > T(0) ? T(1) / s : T(0);
 #pragma unroll
-  for (int k = 0; k < 5; ++k) x[k] = d[k] * inv;
+  for (int k = 0; k < 5; ++k) x[k] = x[k] * inv;
+}
 
-  // forward: h1 = relu(W1 x + b1), z = W3 relu(W2 h1 + b2) + b3 + ln d
-  T h1[MLP_HID];
-  unsigned int m1 = 0, m2 = 0;
+// The network on the cell whose stencil starts at v (in LDS, the same cell in
+// every lane): weights w0, w2 and, of the reconstructed value r = h1 +
+// w0 (h0 - h1) + w2 (h2 - h1), w = softmax(z), the gradient xb with respect to
+// the inputs, back through softmax and the three layers (ReLU masks of this
+// evaluation). The lanes 0 .. 31 are the hidden units of the right side, the
+// lanes 32 .. 63 those of the left side (the mirrored stencil); a layer's
+// values pass through LDS, sums over units through DPP.
+template <typename T>
+__device__ __forceinline__ void learned_network(VjpNet<T, true> &net, const T *s_v, T &p0,
+                                                T &p2, T xb[5]) {
+  const int lane = threadIdx.x & 63;
+  const int unit = lane & 31;
+  const bool left = lane >= 32;
+  T *hb = net.h[threadIdx.x >> 6][left ? 1 : 0];
+  const T v[5] = {s_v[0], s_v[1], s_v[2], s_v[3], s_v[4]};
+  T x[5], inv, sg;
+  int km;
+  learned_inputs(v, x, inv, sg, km);
+  const T D0 = v[1] - v[0], D1 = v[2] - v[1], D2 = v[3] - v[2], D3 = v[4] - v[3];
+  const T s0 = D1 - D0, s1 = D2 - D1, s2 = D3 - D2;
+  const T t0 = s1 - s0, t1 = s2 - s1;
+
+  // forward
+  T w1[MLP_IN], w3[MLP_OUT];
 #pragma unroll
-  for (int j = 0; j < MLP_HID; ++j) {
-    T a = static_cast<T>(P[MLP_B1 + j]);
+  for (int k = 0; k < MLP_IN; ++k) w1[k] = net.w1[unit][k];
 #pragma unroll
-    for (int k = 0; k < MLP_IN; ++k) a = fma(mlp_weight<T>(P, MLP_W1 + j * MLP_IN + k), x[k], a);
-    m1 |= a > T(0) ? (1u << j) : 0u;
-    h1[j] = a > T(0) ? a : T(0);
-  }
+  for (int o = 0; o < MLP_OUT; ++o) w3[o] = net.w3[o][unit];
+  T a1 = net.b1[unit];
+#pragma unroll
+  for (int k = 0; k < 5; ++k) a1 = fma(w1[k], left ? x[4 - k] : x[k], a1);
+  hb[unit] = a1 > T(0) ? a1 : T(0);
+  __builtin_amdgcn_wave_barrier();
+  T acc[4] = {net.b2[unit], T(0), T(0), T(0)};
+#pragma unroll 8
+  for (int j = 0; j < MLP_HID; ++j) acc[j & 3] = fma(net.w2[unit][j], hb[j], acc[j & 3]);
+  const T a2 = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+  const T h2 = a2 > T(0) ? a2 : T(0);
   T z[MLP_OUT];
-  const float lnd[3] = {MLP_LN_D0, MLP_LN_D1, MLP_LN_D2};
 #pragma unroll
-  for (int o = 0; o < MLP_OUT; ++o) z[o] = static_cast<T>(P[MLP_B3 + o] + lnd[o]);
-  // rows of layer 2 one at a time (a rolled loop: the row's 32 weights are
-  // loaded when it runs)
-#pragma unroll 1
-  for (int i = 0; i < MLP_HID; ++i) {
-    T a = static_cast<T>(P[MLP_B2 + i]);
-#pragma unroll
-    for (int j = 0; j < MLP_HID; ++j) a = fma(mlp_weight<T>(P, MLP_W2 + i * MLP_HID + j), h1[j], a);
-    if (a > T(0)) {
-      m2 |= 1u << i;
-#pragma unroll
-      for (int o = 0; o < MLP_OUT; ++o)
-        z[o] = fma(mlp_weight<T>(P, MLP_W3 + o * MLP_HID + i), a, z[o]);
-    }
-  }
+  for (int o = 0; o < MLP_OUT; ++o) z[o] = half_sum(w3[o] * h2) + net.b3[o];
   const T zm = fmax(fmax(z[0], z[1]), z[2]);
   const T e0 = exp(z[0] - zm), e1 = exp(z[1] - zm), e2 = exp(z[2] - zm);
-  const T es = (e0 + e1) + e2;
-  const T w0 = e0 / es, w1 = e1 / es, w2 = e2 / es;
-  T h0c, h1c, h2c;
-  weno_uhat(v0, v1, v2, v3, v4, h0c, h1c, h2c);
-  const T r = (h1c + w0 * (h0c - h1c)) + w2 * (h2c - h1c);
-
-#pragma unroll
-  for (int k = 0; k < 5; ++k) G[k] = T(0);
-  uhat_grad(w0, (T(1) - w0) - w2, w2, G);
+  const T es = T(1) / ((e0 + e1) + e2);
+  p0 = e0 * es;
+  p2 = e2 * es;
+  const T p1 = e1 * es;
 
   // backward: dr/dw = (h0 - h1, 0, h2 - h1), through softmax
-  const T c0 = h0c - h1c, c2 = h2c - h1c;
-  const T sw = c0 * w0 + c2 * w2;
-  const T zb[MLP_OUT] = {w0 * (c0 - sw), w1 * (T(0) - sw), w2 * (c2 - sw)};
-  // h1b = W2^T (mask2 * W3^T zb), then xb = W1^T (mask1 * h1b)
-  T h1b[MLP_HID];
+  const T c0 = left ? t1 * T(1.0 / 3.0) : t0 * T(-1.0 / 3.0);
+  const T c2 = left ? t0 * T(1.0 / 6.0) : t1 * T(-1.0 / 6.0);
+  const T sw = c0 * p0 + c2 * p2;
+  const T hb2 =
+      fma(w3[0], p0 * (c0 - sw), fma(w3[1], p1 * (T(0) - sw), w3[2] * (p2 * (c2 - sw))));
+  __builtin_amdgcn_wave_barrier();
+  hb[unit] = a2 > T(0) ? hb2 : T(0);
+  __builtin_amdgcn_wave_barrier();
+  T bcc[4] = {T(0), T(0), T(0), T(0)};
+#pragma unroll 8
+  for (int i = 0; i < MLP_HID; ++i) bcc[i & 3] = fma(net.w2[i][unit], hb[i], bcc[i & 3]);
+  T hb1 = (bcc[0] + bcc[1]) + (bcc[2] + bcc[3]);
+  hb1 = a1 > T(0) ? hb1 : T(0);
 #pragma unroll
-  for (int j = 0; j < MLP_HID; ++j) h1b[j] = T(0);
-#pragma unroll 1
-  for (int i = 0; i < MLP_HID; ++i) {
-    if (m2 & (1u << i)) {
-      T h2b = T(0);
-#pragma unroll
-      for (int o = 0; o < MLP_OUT; ++o)
-        h2b = fma(mlp_weight<T>(P, MLP_W3 + o * MLP_HID + i), zb[o], h2b);
-#pragma unroll
-      for (int j = 0; j < MLP_HID; ++j)
-        h1b[j] = fma(mlp_weight<T>(P, MLP_W2 + i * MLP_HID + j), h2b, h1b[j]);
-    }
+  for (int k = 0; k < 5; ++k) xb[k] = half_sum(w1[k] * hb1);
+  __builtin_amdgcn_wave_barrier();
+}
+
+// What the network adds to the states of the learned cells of a workgroup:
+// the weights of both sides (into c: wR = (w0, ., w2), wL likewise, mirrored)
+// and the gradients gR, gL of the states through the weights, on the
+// (unmirrored) stencil. s_u: the states, cell t's stencil at s_u[t]; res:
+// kLearnedRound * 14 values of LDS scratch. Ends a barrier after its first
+// reads of net.count.
+//
+// The learned cells sit together around jumps and critical points, ten or
+// twenty of them in one or two waves of a grid. They are collected for the
+// workgroup and dealt to its waves, and a wave evaluates one with a lane per
+// hidden unit: with a lane per cell that walked the network alone, a stage
+// waited for two serial loops over its rows and a reverse step of 16
+// instances of 16384 cells took 377 us.
+constexpr int kLearnedRound = 64;  // cells per round
+
+template <typename T>
+__device__ __forceinline__ void learned_cells_grad(VjpNet<T, true> &net, bool learned,
+                                                   const T *s_u, const T v[5], T *res,
+                                                   CellStates<T> &c, T gR[5], T gL[5]) {
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const unsigned long long mine = __ballot(learned);
+  int slot = 0;
+  if (mine != 0) {  // wave-uniform
+    int base = 0;
+    if (lane == 0) base = atomicAdd(&net.count, __popcll(mine));
+    slot = __builtin_amdgcn_readfirstlane(base) +
+           __popcll(mine & ((1ull << lane) - 1ull));
+    if (learned) net.cell[slot] = static_cast<unsigned short>(tid);
   }
-  T xb[MLP_IN] = {T(0), T(0), T(0), T(0), T(0)};
+  __syncthreads();
+  const int total = __builtin_amdgcn_readfirstlane(net.count);
+  if (total == 0) return;  // workgroup-uniform
+  for (int r0 = 0; r0 < total; r0 += kLearnedRound) {
+    const int end = total - r0 < kLearnedRound ? total - r0 : kLearnedRound;
+    for (int e = tid >> 6; e < end; e += kVjpWaves) {
+      const int cell = __builtin_amdgcn_readfirstlane(net.cell[r0 + e]);
+      T p0, p2, xb[5];
+      learned_network(net, s_u + cell, p0, p2, xb);
+      if ((lane & 31) == 0) {
+        T *out = res + 14 * e + (lane >= 32 ? 7 : 0);
+        out[0] = p0;
+        out[1] = p2;
 #pragma unroll
-  for (int j = 0; j < MLP_HID; ++j) {
-    if (m1 & (1u << j)) {
-#pragma unroll
-      for (int k = 0; k < MLP_IN; ++k)
-        xb[k] = fma(mlp_weight<T>(P, MLP_W1 + j * MLP_IN + k), h1b[j], xb[k]);
+        for (int k = 0; k < 5; ++k) out[2 + k] = xb[k];
+      }
     }
+    __syncthreads();
+    if (learned && slot >= r0 && slot < r0 + end) {
+      const T *in = res + 14 * (slot - r0);
+      c.wR0 = in[0];
+      c.wR2 = in[1];
+      c.wL2 = in[7];
+      c.wL0 = in[8];
+#pragma unroll
+      for (int k = 0; k < 5; ++k) {
+        gR[k] = in[2 + k];
+        gL[k] = in[13 - k];  // back on the unmirrored stencil
+      }
+    }
+    if (r0 + kLearnedRound < total) __syncthreads();
   }
-  if (s > T(0)) {
-    // x_k = d_k / s: dx_k/dv_j = (delta_kj - 1/5) / s - x_k sgn(d_km)
-    // (delta_km,j - 1/5) / s
-    T sxb = T(0), dot = T(0);
+
+  // from the inputs to the stencil: x_k = d_k / s with d = v - mean and s =
+  // |d_km|: dx_k/dv_j = (delta_kj - 1/5) / s - x_k sgn(d_km) (delta_km,j - 1/5) / s
+  if (learned) {
+    T x[5], inv, sg;
+    int km;
+    learned_inputs(v, x, inv, sg, km);
+    T sr = T(0), sl = T(0), dr = T(0), dl = T(0);
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
-      sxb += xb[k];
-      dot += xb[k] * x[k];
+      sr += gR[k];
+      sl += gL[k];
+      dr += gR[k] * x[k];
+      dl += gL[k] * x[k];
     }
-    const T sg = d[km] > T(0) ? T(1) : T(-1);
 #pragma unroll
     for (int j = 0; j < 5; ++j) {
       const T ds = sg * ((j == km ? T(1) : T(0)) - T(0.2));
-      G[j] += inv * ((xb[j] - T(0.2) * sxb) - dot * ds);
+      gR[j] = inv * ((gR[j] - T(0.2) * sr) - dr * ds);
+      gL[j] = inv * ((gL[j] - T(0.2) * sl) - dl * ds);
     }
   }
-  return r;
 }
 
-// Scratch of one reverse stage over a block of B computing cells.
-template <typename T, bool SPLIT = true>
+// Scratch of one reverse stage over a block of kVjpBlock computing cells.
+template <typename T, bool LEARNED>
 struct VjpScratch {
-  T ur[kVjpBlock], ul[kVjpBlock];
-  T cR[kVjpBlock], cL[kVjpBlock], sL[kVjpBlock], sR[kVjpBlock];
+  T ul[kVjpBlock];
+  T cL[kVjpBlock], sR[kVjpBlock];
   T P[5][kVjpBlock];
-  // gradients of the left reconstructions (computed by the other half of a
-  // split block)
-  T GL[SPLIT ? 5 : 1][SPLIT ? kVjpBlock : 1];
+  VjpNet<T, LEARNED> net;
 };
 
 // JL(state)^T mu for the output cells Z .. Z + B - 7 of one block: s_u holds
 // the state at cells Z - 5 .. Z + B - 2, s_mu the cotangent at Z - 3 ..
-// Z + B - 3 (both in LDS, visible to the block). SPLIT (2 B threads): thread
-// t < B computes the right reconstruction of cell Z - 3 + t and its
-// gradient, thread B + t the left one (the two chains side by side, for
-// grids too small to fill the device); otherwise (B threads) thread t
-// computes both. Thread t returns the gathered sum of output cell Z + t
-// (valid for t < B - 6; threads B .. 2 B - 1 return 0). Both forms compute
-// the same values with the same roundings. s_u is read only before the
-// second barrier (a caller may overwrite it once this returns). Ends with
-// the scratch in use.
-template <typename T, int FLUX, bool LEARNED = false, bool SPLIT = true>
+// Z + B - 3 (both in LDS, visible to the block). Thread t computes both
+// reconstructions of cell Z - 3 + t, the face to its right, and its
+// contributions to the five cells around it; it returns the gathered sum of
+// output cell Z + t (valid for t < B - 6). s_u is read only before the second
+// barrier (a caller may overwrite it once this returns). Ends with the scratch
+// in use.
+//
+// VALU-bound in a batch, latency-bound for one instance. Both sides in one
+// thread share the indicators and reciprocals, and their gradients are expanded
+// to the stencil once, after the faces have given both cotangents; two threads
+// per cell with a gradient each took 49.7 us (in one thread; 64 instances of
+// 16384 cells) and 7.96 us (in two; one instance) per reverse step.
+template <typename T, int FLUX, bool LEARNED = false>
 __device__ __forceinline__ T vjp_block(const VjpArgs<T> &p, const T *s_u,
-                                       const T *s_mu, VjpScratch<T, SPLIT> &sc) {
+                                       const T *s_mu, VjpScratch<T, LEARNED> &sc) {
   constexpr int B = kVjpBlock;
   const int tid = threadIdx.x;
-  const bool left = SPLIT && tid >= B;
-  const int c = left ? tid - B : tid;
 
-  // ---- one reconstruction of computing cell Z - 3 + c and its gradient:
-  // the right one from v0 .. v4, the left one from the mirrored stencil
-  T G[5];
-  const T v0 = s_u[c], v1 = s_u[c + 1], v2 = s_u[c + 2], v3 = s_u[c + 3], v4 = s_u[c + 4];
-  const T w0 = left ? v4 : v0, w1 = left ? v3 : v1, w3 = left ? v1 : v3,
-          w4 = left ? v0 : v4;
-  T rec;
+  // ---- both states of computing cell Z - 3 + tid
+  const T v[5] = {s_u[tid], s_u[tid + 1], s_u[tid + 2], s_u[tid + 3], s_u[tid + 4]};
+  CellStates<T> c;
+  T ul, ur;
+  int regime = 0;
+  T gR[LEARNED ? 5 : 1] = {}, gL[LEARNED ? 5 : 1] = {};
   if constexpr (LEARNED) {
-    const int regime = learned_regime5(v0, v1, v2, v3, v4, p.eps4, p.tau, p.sigma);
-    if (regime == 0) {
-      rec = weno_side_grad(w0, w1, v2, w3, w4, p.eps, G);
-    } else if (regime == 1) {
-      rec = ideal_side_grad(w0, w1, v2, w3, w4, G);
-    } else {
-      rec = learned_side_grad(p.mlp, w0, w1, v2, w3, w4, G);
-    }
+    // the forward kernels' regime, from their arithmetic (reconstruct_cells)
+    using C = Weno5Coeffs<T>;
+    T D1, D2, e[3];
+    weno_cell_indicators(v, p.eps4, D1, D2, c, e);
+    regime = mlp_regime(fma(c.t[0], c.t[0], C::a0x4 * (c.s[0] * c.s[0])),
+                        fma(c.t[1], c.t[1], C::a0x4 * (c.s[1] * c.s[1])),
+                        fma(c.t[2], c.t[2], C::a0x4 * (c.s[2] * c.s[2])), p.eps4, p.tau,
+                        p.sigma);
+    c.wR0 = c.wL2 = T(0.1);
+    c.wR2 = c.wL0 = T(0.3);
+    static_assert(5 * B >= 14 * kLearnedRound, "the scatter's scratch holds a round");
+    learned_cells_grad(sc.net, regime == 2, s_u, v, &sc.P[0][0], c, gR, gL);
+    T mR, mL;
+    weno_cell_values(v[2], D1, D2, c, mR, mL, ul, ur);
+    if (regime == 0) weno_cell_states(v, p.eps4, c, ul, ur);
   } else {
-    rec = weno_side_grad(w0, w1, v2, w3, w4, p.eps, G);
+    weno_cell_states(v, p.eps4, c, ul, ur);
   }
-  if constexpr (SPLIT) {
-    if (left) {
-      sc.ul[c] = rec;
-#pragma unroll
-      for (int k = 0; k < 5; ++k) sc.GL[k][c] = G[k];
-    } else {
-      sc.ur[c] = rec;
-    }
-  } else {
-    sc.ur[c] = rec;
-  }
-  T GLm[5];
-  if constexpr (!SPLIT) {
-    // the left reconstruction in the same thread, kept in registers
-    T recl;
-    if constexpr (LEARNED) {
-      const int regime = learned_regime5(v0, v1, v2, v3, v4, p.eps4, p.tau, p.sigma);
-      if (regime == 0) {
-        recl = weno_side_grad(v4, v3, v2, v1, v0, p.eps, GLm);
-      } else if (regime == 1) {
-        recl = ideal_side_grad(v4, v3, v2, v1, v0, GLm);
-      } else {
-        recl = learned_side_grad(p.mlp, v4, v3, v2, v1, v0, GLm);
-      }
-    } else {
-      recl = weno_side_grad(v4, v3, v2, v1, v0, p.eps, GLm);
-    }
-    sc.ul[c] = recl;
-  }
-  if (tid == 0) {
-    sc.cL[0] = T(0);
-    sc.sR[0] = T(0);
-  }
+  sc.ul[tid] = ul;
   __syncthreads();
+  if constexpr (LEARNED) {
+    // (the next stage adds to it after the barriers below)
+    if (tid == 0) sc.net.count = 0;
+  }
 
-  // ---- face c + 1/2: cotangent of the flux and its partial derivatives
+  // ---- the face right of the cell: cotangent of the flux and its partial
+  // derivatives (cR, sL stay here, cL and sR go to the next cell)
+  T cR = T(0), sL = T(0);
   if (tid < B - 1) {
-    const T urL = sc.ur[tid], ulR = sc.ul[tid + 1];
-    const T uL = s_u[tid + 2], uR = s_u[tid + 3];
+    const T urL = ur, ulR = sc.ul[tid + 1];
+    const T uL = v[2], uR = v[3];
     T gF = (s_mu[tid + 1] - s_mu[tid]) * p.inv_dx;
     T dur = T(0), dul = T(0), duL = T(0), duR = T(0);
     if constexpr (FLUX == PSA_FLUX_RUSANOV) {
@@ -485,27 +634,27 @@ __device__ __forceinline__ T vjp_block(const VjpArgs<T> &p, const T *s_u,
         dul = T(1);
       }
     }
-    sc.cR[tid] = gF * dur;
+    cR = gF * dur;
+    sL = gF * duL;
     sc.cL[tid + 1] = gF * dul;
-    sc.sL[tid] = gF * duL;
-    sc.sR[tid + 1] = gF * duR;
+    if constexpr (FLUX == PSA_FLUX_RUSANOV) sc.sR[tid + 1] = gF * duR;
   }
   __syncthreads();
 
-  // ---- scatter: contribution of cell c's reconstructions to c - 2 .. c + 2
+  // ---- contributions of the cell to c - 2 .. c + 2
   if (tid >= 1 && tid <= B - 2) {
-    const T cR = sc.cR[tid], cL = sc.cL[tid];
-    // (one explicit multiply-add, so that both forms round alike)
+    const T cL = sc.cL[tid];
+    T P[5];
+    weno_cell_scatter(c, cR, cL, LEARNED && regime != 0, P);
+    if constexpr (LEARNED) {
+      if (regime == 2) {
 #pragma unroll
-    for (int r = 0; r < 5; ++r) {
-      T gl;
-      if constexpr (SPLIT) {
-        gl = sc.GL[4 - r][tid];
-      } else {
-        gl = GLm[4 - r];
+        for (int r = 0; r < 5; ++r) P[r] += fma(cR, gR[r], cL * gL[r]);
       }
-      sc.P[r][tid] = fma(cR, G[r], cL * gl);
     }
+    if constexpr (FLUX == PSA_FLUX_RUSANOV) P[2] += sL + sc.sR[tid];
+#pragma unroll
+    for (int r = 0; r < 5; ++r) sc.P[r][tid] = P[r];
   }
   __syncthreads();
 
@@ -513,7 +662,6 @@ __device__ __forceinline__ T vjp_block(const VjpArgs<T> &p, const T *s_u,
   T gsum = T(0);
   if (tid < B - 6) {
     const int q = tid + 3;
-    gsum = (sc.sL[q] + sc.sR[q]);
 #pragma unroll
     for (int r = 0; r < 5; ++r) gsum += sc.P[r][q + 2 - r];
   }
@@ -538,11 +686,11 @@ __device__ __forceinline__ T vjp_value(T mu, T gsum, T dt, T lam, T lamk2) {
 // RSTAGE 0: out = JL(state)^T mu; 3, 2, 1: the reverse stages above, with
 // mu = l, lk2, lk1 respectively.
 template <typename T, int FLUX, int RSTAGE, bool LEARNED = false>
-__global__ __launch_bounds__(kVjpThreads) void k_stage_vjp(VjpArgs<T> p) {
+__global__ __launch_bounds__(kVjpBlock) void k_stage_vjp(VjpArgs<T> p) {
   constexpr int B = kVjpBlock;
   __shared__ T s_u[B + 4];   // cells S - 5 ..
   __shared__ T s_mu[B + 1];  // cells S - 3 ..
-  __shared__ VjpScratch<T> sc;
+  __shared__ VjpScratch<T, LEARNED> sc;
 
   const int tid = threadIdx.x;
   const int64_t n = p.n;
@@ -559,10 +707,10 @@ __global__ __launch_bounds__(kVjpThreads) void k_stage_vjp(VjpArgs<T> p) {
     p.out[p.m - g + tid] = T(0);
   }
 
-  for (int j = tid; j < B + 4; j += kVjpThreads)
-    s_u[j] = load_periodic(p.state, S - 5 + j, n, g);
-  for (int j = tid; j < B + 1; j += kVjpThreads)
-    s_mu[j] = load_periodic(p.mu, S - 3 + j, n, g);
+  if constexpr (LEARNED) vjp_net_load(sc.net, p.mlp);
+  const PeriodicSpan cu(S - 5, n, g), cm(S - 3, n, g);
+  for (int j = tid; j < B + 4; j += B) s_u[j] = cu.load(p.state, j);
+  for (int j = tid; j < B + 1; j += B) s_mu[j] = cm.load(p.mu, j);
   __syncthreads();
 
   const T gsum = vjp_block<T, FLUX, LEARNED>(p, s_u, s_mu, sc);
@@ -590,6 +738,11 @@ struct StepVjpArgs {
                     //   bstride of every array, its dt at dt_ptr[blockIdx.y]
 };
 
+// Waves per SIMD the registers of the plain reverse step are kept within.
+#ifndef PSA_VJP_WAVES
+#define PSA_VJP_WAVES 5
+#endif
+
 constexpr int kStepVjpOut = kVjpBlock - 18;  // output cells per workgroup
 
 // The three reverse stages of one step in one pass: a workgroup loads k2,
@@ -597,19 +750,17 @@ constexpr int kStepVjpOut = kVjpBlock - 18;  // output cells per workgroup
 // reverse stages 3, 2 and 1 in LDS (vjp_block each): lk2 is exact on
 // [S - 6, S + B - 12), lk1 on [S - 3, S + B - 15), the step's cotangent on the
 // output cells [S, S + B - 18). The same arithmetic as k_stage_vjp.
-template <typename T, int FLUX, bool LEARNED = false, bool SPLIT = true>
-__global__ __launch_bounds__(SPLIT ? kVjpThreads : kVjpBlock)
-__attribute__((amdgpu_waves_per_eu(SPLIT || LEARNED ? 1 : 5))) void k_step_vjp(
+template <typename T, int FLUX, bool LEARNED = false>
+__global__ __launch_bounds__(kVjpBlock)
+__attribute__((amdgpu_waves_per_eu(LEARNED ? 3 : PSA_VJP_WAVES))) void k_step_vjp(
     StepVjpArgs<T> a) {
   constexpr int B = kVjpBlock;
-  constexpr int NT = SPLIT ? kVjpThreads : kVjpBlock;
   __shared__ T sK2[B + 4], sK1[B + 4], sX[B + 4];
   __shared__ T sLam[B + 4];  // cells S - 9 ..
-  __shared__ VjpScratch<T, SPLIT> sc;
+  __shared__ VjpScratch<T, LEARNED> sc;
   // lk2 (cells S - 6 ..) takes k2's buffer and lk1 (cells S - 3 ..) k1's:
   // each is written once the reverse stage that reads that state has
   // returned, and vjp_block reads its state only before its second barrier
-  // (4 KB less LDS: one more workgroup per CU for the one-thread form)
   T *const sLk2 = sK2;
   T *const sLk1 = sK1;
   const VjpArgs<T> &p = a.v;
@@ -629,28 +780,30 @@ __attribute__((amdgpu_waves_per_eu(SPLIT || LEARNED ? 1 : 5))) void k_step_vjp(
     xout[tid] = T(0);
     xout[p.m - g + tid] = T(0);
   }
-  for (int j = tid; j < B + 4; j += NT) {
-    sK2[j] = load_periodic(xk2, S - 11 + j, n, g);
-    sK1[j] = load_periodic(xk1, S - 8 + j, n, g);
-    sX[j] = load_periodic(xx, S - 5 + j, n, g);
-    sLam[j] = load_periodic(xlam, S - 9 + j, n, g);
+  if constexpr (LEARNED) vjp_net_load(sc.net, p.mlp);
+  const PeriodicSpan c2(S - 11, n, g), c1(S - 8, n, g), cx(S - 5, n, g), cl(S - 9, n, g);
+  for (int j = tid; j < B + 4; j += B) {
+    sK2[j] = c2.load(xk2, j);
+    sK1[j] = c1.load(xk1, j);
+    sX[j] = cx.load(xx, j);
+    sLam[j] = cl.load(xlam, j);
   }
   __syncthreads();
 
   // reverse stage 3 on the output cells S - 6 + t: lk2 (with zeros in the
   // entries past the exact cotangents, read only for cells outside the exact
   // ranges: finite values)
-  T gsum = vjp_block<T, FLUX, LEARNED, SPLIT>(p, sK2, sLam, sc);
+  T gsum = vjp_block<T, FLUX, LEARNED>(p, sK2, sLam, sc);
   if (tid < B - 6) sLk2[tid] = vjp_value<T, 3>(sLam[tid + 3], gsum, dt, T(0), T(0));
   for (int j = B - 6 + tid; j < B + 1; j += B) sLk2[j] = T(0);
   __syncthreads();
   // reverse stage 2 on S - 3 + t: lk1
-  gsum = vjp_block<T, FLUX, LEARNED, SPLIT>(p, sK1, sLk2, sc);
+  gsum = vjp_block<T, FLUX, LEARNED>(p, sK1, sLk2, sc);
   if (tid < B - 6) sLk1[tid] = vjp_value<T, 2>(sLk2[tid + 3], gsum, dt, T(0), T(0));
   for (int j = B - 6 + tid; j < B + 1; j += B) sLk1[j] = T(0);
   __syncthreads();
   // reverse stage 1 on S + t: the cotangent of the step input
-  gsum = vjp_block<T, FLUX, LEARNED, SPLIT>(p, sX, sLk1, sc);
+  gsum = vjp_block<T, FLUX, LEARNED>(p, sX, sLk1, sc);
   if (tid < kStepVjpOut) {
     const int64_t j = S + tid;
     if (j < p.m - g)
@@ -728,13 +881,15 @@ __global__ __launch_bounds__(kLfBlock) void k_lf_speed_vjp(VjpArgs<T> p) {
   // G over the n faces of the periodic ring (face j between cells j - 1, j)
   T acc = T(0);
   for (int64_t j = g + tid; j < m - g; j += kLfBlock) {
+    const PeriodicSpan span(j - 3, n, g);
     T v[6];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) v[k] = load_periodic(p.state, j - 3 + k, n, g);
-    T G[5];
-    const T urL = weno_side_grad(v[0], v[1], v[2], v[3], v[4], p.eps, G);
-    const T ulR = weno_side_grad(v[5], v[4], v[3], v[2], v[1], p.eps, G);
-    const T gF = (load_periodic(p.mu, j, n, g) - load_periodic(p.mu, j - 1, n, g)) * p.inv_dx;
+    for (int k = 0; k < 6; ++k) v[k] = span.load(p.state, k);
+    CellStates<T> c;
+    T urL, ulR, unused;
+    weno_cell_states(v, p.eps4, c, unused, urL);
+    weno_cell_states(v + 1, p.eps4, c, ulR, unused);
+    const T gF = (span.load(p.mu, 3) - span.load(p.mu, 2)) * p.inv_dx;
     acc += gF * (T(-0.5) * (ulR - urL));
   }
   const T G = lf_block_sum(acc, s_red);
@@ -777,19 +932,19 @@ int launch_vjp_flux(int rstage, const VjpArgs<T> &a, hipStream_t s) {
   switch (rstage) {
     case 0:
       hipLaunchKernelGGL((k_stage_vjp<T, FLUX, 0, LEARNED>), dim3(blocks),
-                         dim3(kVjpThreads), 0, s, a);
+                         dim3(kVjpBlock), 0, s, a);
       break;
     case 1:
       hipLaunchKernelGGL((k_stage_vjp<T, FLUX, 1, LEARNED>), dim3(blocks),
-                         dim3(kVjpThreads), 0, s, a);
+                         dim3(kVjpBlock), 0, s, a);
       break;
     case 2:
       hipLaunchKernelGGL((k_stage_vjp<T, FLUX, 2, LEARNED>), dim3(blocks),
-                         dim3(kVjpThreads), 0, s, a);
+                         dim3(kVjpBlock), 0, s, a);
       break;
     default:
       hipLaunchKernelGGL((k_stage_vjp<T, FLUX, 3, LEARNED>), dim3(blocks),
-                         dim3(kVjpThreads), 0, s, a);
+                         dim3(kVjpBlock), 0, s, a);
       break;
   }
   return check_launch("stage vjp");
@@ -854,29 +1009,6 @@ int launch_vjp(const psa_solver_desc *d, int rstage, const void *state,
   return launch_vjp_flux<T, PSA_FLUX_ADVECTION_UPWIND>(rstage, a, s);
 }
 
-// Grids of at most this many workgroups run the split reverse step.
-constexpr long long kVjpSplitMaxBlocks = 512;
-
-template <typename T, bool SPLIT>
-int launch_step_vjp_plain(const psa_solver_desc *d, dim3 grid, const StepVjpArgs<T> &a,
-                          hipStream_t s) {
-  const dim3 block(SPLIT ? kVjpThreads : kVjpBlock);
-  if (d->flux == PSA_FLUX_RUSANOV) {
-    hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_RUSANOV, false, SPLIT>), grid, block, 0, s,
-                       a);
-  } else if (d->flux == PSA_FLUX_BURGERS_UPWIND) {
-    hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_BURGERS_UPWIND, false, SPLIT>), grid, block,
-                       0, s, a);
-  } else if (d->flux == PSA_FLUX_ENGQUIST_OSHER) {
-    hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_ENGQUIST_OSHER, false, SPLIT>), grid, block,
-                       0, s, a);
-  } else {
-    hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_ADVECTION_UPWIND, false, SPLIT>), grid,
-                       block, 0, s, a);
-  }
-  return check_launch("step vjp");
-}
-
 // The three reverse stages of one step as one launch (k_step_vjp).
 template <typename T>
 int launch_step_vjp(const psa_solver_desc *d, const void *x, const void *k1,
@@ -902,25 +1034,27 @@ int launch_step_vjp(const psa_solver_desc *d, const void *x, const void *k1,
   a.out = static_cast<T *>(out);
   const dim3 grid(static_cast<unsigned int>((d->n + kStepVjpOut - 1) / kStepVjpOut),
                   static_cast<unsigned int>(batch));
+  const dim3 block(kVjpBlock);
   if (d->mlp != nullptr) {
     if (d->flux == PSA_FLUX_RUSANOV) {
-      hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_RUSANOV, true>), grid, dim3(kVjpThreads), 0,
-                         s, a);
+      hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_RUSANOV, true>), grid, block, 0, s, a);
     } else if (d->flux == PSA_FLUX_ENGQUIST_OSHER) {
-      hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_ENGQUIST_OSHER, true>), grid,
-                         dim3(kVjpThreads), 0, s, a);
+      hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_ENGQUIST_OSHER, true>), grid, block, 0, s,
+                         a);
     } else {
-      hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_BURGERS_UPWIND, true>), grid,
-                         dim3(kVjpThreads), 0, s, a);
+      hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_BURGERS_UPWIND, true>), grid, block, 0, s,
+                         a);
     }
-    return check_launch("learned step vjp");
+  } else if (d->flux == PSA_FLUX_RUSANOV) {
+    hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_RUSANOV>), grid, block, 0, s, a);
+  } else if (d->flux == PSA_FLUX_BURGERS_UPWIND) {
+    hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_BURGERS_UPWIND>), grid, block, 0, s, a);
+  } else if (d->flux == PSA_FLUX_ENGQUIST_OSHER) {
+    hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_ENGQUIST_OSHER>), grid, block, 0, s, a);
+  } else {
+    hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_ADVECTION_UPWIND>), grid, block, 0, s, a);
   }
-  // a grid that leaves the device short of waves splits each cell's two
-  // reconstructions between two threads (latency); a larger one keeps them
-  // in one thread (throughput)
-  if (static_cast<long long>(grid.x) * grid.y <= kVjpSplitMaxBlocks)
-    return launch_step_vjp_plain<T, true>(d, grid, a, s);
-  return launch_step_vjp_plain<T, false>(d, grid, a, s);
+  return check_launch("step vjp");
 }
 
 int check_vjp_desc(const psa_solver_desc *d) {
