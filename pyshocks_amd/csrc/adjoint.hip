@@ -38,6 +38,7 @@
 #include "../../include/pyshocks_amd.h"
 #include "mlp_device.hpp"
 #include "psa_internal.hpp"
+#include "stage_device.hpp"
 #include "weno5_device.hpp"
 
 namespace psa {
@@ -46,36 +47,7 @@ namespace {
 constexpr int kVjpBlock = 256;          // threads and computing cells per workgroup
 constexpr int kVjpWaves = kVjpBlock / 64;
 constexpr int kVjpOut = kVjpBlock - 6;  // output cells per workgroup
-
-// The cells first, first + 1, .. of a periodic array with n interior cells and
-// g ghosts, first >= g - n (in [g - n, g + n) but for the tiniest grids). A
-// subtraction for each index instead of a 64-bit remainder, which cost as
-// much as a reverse stage.
-struct PeriodicSpan {
-  int64_t lo;  // the first cell's interior index, in [0, n)
-  int64_t n;
-  int g;
-
-  __device__ __forceinline__ PeriodicSpan(int64_t first, int64_t n_, int g_)
-      : n(n_), g(g_) {
-    int64_t k = first - g_;
-    if (k < 0) {
-      k += n;
-      if (k < 0) k = k % n + n;
-    }
-    if (k >= n) k %= n;
-    lo = k;
-  }
-  template <typename T>
-  __device__ __forceinline__ T load(const T *__restrict__ u, int j) const {
-    int64_t k = lo + j;
-    if (k >= n) {
-      k -= n;
-      if (k >= n) k %= n;
-    }
-    return u[g + k];
-  }
-};
+constexpr int kVjpMostSteps = 12;       // reverse steps of a launch (40 output cells)
 
 // 1 / x for a positive normal FP64 x: the hardware reciprocal y (relative
 // error e below 1e-7) with e + e^2 added, which leaves e^3.
@@ -725,17 +697,19 @@ __global__ __launch_bounds__(kVjpBlock) void k_stage_vjp(VjpArgs<T> p) {
   }
 }
 
-// Arguments of the fused reverse step.
+// Arguments of the fused reverse steps.
 template <typename T>
 struct StepVjpArgs {
-  VjpArgs<T> v;     // eps, inv_dx, vconst, dt_ptr, m, n, g
-  const T *x;       // the step's input state
+  VjpArgs<T> v;     // eps4, inv_dx, vconst, dt_ptr, m, n, g
+  const T *x;       // the input state of the last step (the first one reversed)
   const T *k1;      // its stage states
   const T *k2;
-  const T *lam;     // cotangent of the step output
-  T *out;           // cotangent of the step input
+  const T *lam;     // cotangent of that step's output
+  T *out;           // cotangent of the input of the first step
+  int64_t stride;   // from a step's states back to those of the step before
   int64_t bstride;  // a batch: instance blockIdx.y at offset blockIdx.y *
                     //   bstride of every array, its dt at dt_ptr[blockIdx.y]
+  int nsub;         // steps reversed by the launch
 };
 
 // Waves per SIMD the registers of the plain reverse step are kept within.
@@ -743,16 +717,27 @@ struct StepVjpArgs {
 #define PSA_VJP_WAVES 5
 #endif
 
-constexpr int kStepVjpOut = kVjpBlock - 18;  // output cells per workgroup
+// Output cells per workgroup of nsub reverse steps.
+constexpr int step_vjp_out(int nsub) { return kVjpBlock - 18 * nsub; }
 
-// The three reverse stages of one step in one pass: a workgroup loads k2,
-// k1, x and the incoming cotangent with halos of 11, 8, 5 and 9 cells and runs
-// reverse stages 3, 2 and 1 in LDS (vjp_block each): lk2 is exact on
-// [S - 6, S + B - 12), lk1 on [S - 3, S + B - 15), the step's cotangent on the
-// output cells [S, S + B - 18). The same arithmetic as k_stage_vjp.
-template <typename T, int FLUX, bool LEARNED = false>
+// nsub reverse steps in one pass: a workgroup loads k2, k1, x and the incoming
+// cotangent with halos of 11, 8, 5 and 9 cells around its window and runs
+// reverse stages 3, 2 and 1 in LDS (vjp_block each). With the window's first
+// cell S: lk2 is exact on [S - 6, S + B - 12), lk1 on [S - 3, S + B - 15), the
+// step's cotangent on [S, S + B - 18); it is the next step's incoming
+// cotangent, whose window starts 9 cells further in, so every step leaves 18
+// cells fewer and the neighbouring workgroups recompute the margins. The same
+// arithmetic as k_stage_vjp, and the same bits whatever nsub.
+//
+// One step per launch is mostly launch, load and drain at the size of a single
+// gradient (N = 16384: 6.3 us a step, 3.1 of them the three stages), on a device that is nearly idle;
+// several share that cost, and the next step's states are loaded while this
+// one computes.
+// MANY: more than one step (the registers of the states in flight, 90 instead
+// of 66, would cost a batch a workgroup per CU).
+template <typename T, int FLUX, bool LEARNED, bool MANY>
 __global__ __launch_bounds__(kVjpBlock)
-__attribute__((amdgpu_waves_per_eu(LEARNED ? 3 : PSA_VJP_WAVES))) void k_step_vjp(
+__attribute__((amdgpu_waves_per_eu(LEARNED ? (MANY ? 2 : 3) : PSA_VJP_WAVES))) void k_step_vjp(
     StepVjpArgs<T> a) {
   constexpr int B = kVjpBlock;
   __shared__ T sK2[B + 4], sK1[B + 4], sX[B + 4];
@@ -767,13 +752,16 @@ __attribute__((amdgpu_waves_per_eu(LEARNED ? 3 : PSA_VJP_WAVES))) void k_step_vj
   const int tid = threadIdx.x;
   const int64_t n = p.n;
   const int g = p.g;
-  const int64_t S = g + static_cast<int64_t>(blockIdx.x) * kStepVjpOut;
+  const int nsub = MANY ? a.nsub : 1;
+  const int nout = step_vjp_out(nsub);
+  // the workgroup's output cells start at A, the first step's window at S
+  const int64_t A = g + static_cast<int64_t>(blockIdx.x) * nout;
+  const int64_t S = A - 9 * (nsub - 1);
   const int64_t off = static_cast<int64_t>(blockIdx.y) * a.bstride;
   const T dt = p.dt_ptr[blockIdx.y];
   const T *xk2 = a.k2 + off;
   const T *xk1 = a.k1 + off;
   const T *xx = a.x + off;
-  const T *xlam = a.lam + off;
   T *xout = a.out + off;
 
   if (blockIdx.x == 0 && tid < g) {
@@ -781,33 +769,70 @@ __attribute__((amdgpu_waves_per_eu(LEARNED ? 3 : PSA_VJP_WAVES))) void k_step_vj
     xout[p.m - g + tid] = T(0);
   }
   if constexpr (LEARNED) vjp_net_load(sc.net, p.mlp);
-  const PeriodicSpan c2(S - 11, n, g), c1(S - 8, n, g), cx(S - 5, n, g), cl(S - 9, n, g);
-  for (int j = tid; j < B + 4; j += B) {
-    sK2[j] = c2.load(xk2, j);
-    sK1[j] = c1.load(xk1, j);
-    sX[j] = cx.load(xx, j);
-    sLam[j] = cl.load(xlam, j);
+  // cells S - 11 + j of the periodic array
+  const PeriodicSpan span(S - 11, n, g);
+  const bool more = tid < 4;
+  {
+    const T *xlam = a.lam + off;
+    for (int j = tid; j < B + 4; j += B) {
+      sK2[j] = span.load(xk2, j);
+      sK1[j] = span.load(xk1, j + 3);
+      sX[j] = span.load(xx, j + 6);
+      sLam[j] = span.load(xlam, j + 2);
+    }
   }
   __syncthreads();
 
-  // reverse stage 3 on the output cells S - 6 + t: lk2 (with zeros in the
-  // entries past the exact cotangents, read only for cells outside the exact
-  // ranges: finite values)
-  T gsum = vjp_block<T, FLUX, LEARNED>(p, sK2, sLam, sc);
-  if (tid < B - 6) sLk2[tid] = vjp_value<T, 3>(sLam[tid + 3], gsum, dt, T(0), T(0));
-  for (int j = B - 6 + tid; j < B + 1; j += B) sLk2[j] = T(0);
-  __syncthreads();
-  // reverse stage 2 on S - 3 + t: lk1
-  gsum = vjp_block<T, FLUX, LEARNED>(p, sK1, sLk2, sc);
-  if (tid < B - 6) sLk1[tid] = vjp_value<T, 2>(sLk2[tid + 3], gsum, dt, T(0), T(0));
-  for (int j = B - 6 + tid; j < B + 1; j += B) sLk1[j] = T(0);
-  __syncthreads();
-  // reverse stage 1 on S + t: the cotangent of the step input
-  gsum = vjp_block<T, FLUX, LEARNED>(p, sX, sLk1, sc);
-  if (tid < kStepVjpOut) {
-    const int64_t j = S + tid;
-    if (j < p.m - g)
-      xout[j] = vjp_value<T, 1>(sLk1[tid + 3], gsum, dt, sLam[tid + 9], sLk2[tid + 6]);
+  for (int s = 0; s < nsub; ++s) {
+    // the next step's states (window 9 cells further in)
+    const bool next = MANY && s + 1 < nsub;
+    T n2 = T(0), n1 = T(0), nx = T(0), e2 = T(0), e1 = T(0), ex = T(0);
+    if (next) {
+      const int64_t back = (s + 1) * a.stride;
+      const int j = tid + 9 * (s + 1);
+      n2 = span.load(xk2 - back, j);
+      n1 = span.load(xk1 - back, j + 3);
+      nx = span.load(xx - back, j + 6);
+      if (more) {
+        e2 = span.load(xk2 - back, j + B);
+        e1 = span.load(xk1 - back, j + B + 3);
+        ex = span.load(xx - back, j + B + 6);
+      }
+    }
+    // reverse stage 3 on the output cells S - 6 + t: lk2 (with zeros in the
+    // entries past the exact cotangents, read only for cells outside the exact
+    // ranges: finite values)
+    T gsum = vjp_block<T, FLUX, LEARNED>(p, sK2, sLam, sc);
+    sLk2[tid] = tid < B - 6 ? vjp_value<T, 3>(sLam[tid + 3], gsum, dt, T(0), T(0)) : T(0);
+    if (tid == 0) sLk2[B] = T(0);
+    __syncthreads();
+    // reverse stage 2 on S - 3 + t: lk1
+    gsum = vjp_block<T, FLUX, LEARNED>(p, sK1, sLk2, sc);
+    sLk1[tid] = tid < B - 6 ? vjp_value<T, 2>(sLk2[tid + 3], gsum, dt, T(0), T(0)) : T(0);
+    if (tid == 0) sLk1[B] = T(0);
+    __syncthreads();
+    // reverse stage 1 on S + t: the cotangent of the step input
+    gsum = vjp_block<T, FLUX, LEARNED>(p, sX, sLk1, sc);
+    const T lam = tid < B - 18 ? vjp_value<T, 1>(sLk1[tid + 3], gsum, dt, sLam[tid + 9],
+                                                 sLk2[tid + 6])
+                               : T(0);
+    if (!next) {
+      const int64_t j = A + tid;
+      if (tid < nout && j < p.m - g) xout[j] = lam;
+      break;
+    }
+    __syncthreads();
+    sLam[tid] = lam;
+    sK2[tid] = n2;
+    sK1[tid] = n1;
+    sX[tid] = nx;
+    if (more) {
+      sLam[B + tid] = T(0);
+      sK2[B + tid] = e2;
+      sK1[B + tid] = e1;
+      sX[B + tid] = ex;
+    }
+    __syncthreads();
   }
 }
 
@@ -1009,13 +1034,56 @@ int launch_vjp(const psa_solver_desc *d, int rstage, const void *state,
   return launch_vjp_flux<T, PSA_FLUX_ADVECTION_UPWIND>(rstage, a, s);
 }
 
-// The three reverse stages of one step as one launch (k_step_vjp).
+// Reverse steps that a launch best takes. Measured (FP64, Rusanov; us a step
+// with 1 step per launch and with the chosen number): one instance of 256 cells
+// 5.33 -> 3.41, of 16384 6.31 -> 3.41, of 65536 7.19 -> 4.48; 16 instances of
+// 16384 11.6 -> 9.5.
+int reverse_steps_per_launch(const psa_solver_desc *d, long long batch) {
+  return best_steps(StepCost{3.3, 2.0, 1.0}, kVjpMostSteps, [&](int k) {
+    const int nout = step_vjp_out(k);
+    return (d->n + nout - 1) / nout * batch;
+  });
+}
+
+template <typename T, bool MANY>
+void launch_step_vjp_flux(const psa_solver_desc *d, const StepVjpArgs<T> &a, dim3 grid,
+                          hipStream_t s) {
+  const dim3 block(kVjpBlock);
+  if (d->mlp != nullptr) {
+    if (d->flux == PSA_FLUX_RUSANOV) {
+      hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_RUSANOV, true, MANY>), grid, block, 0, s, a);
+    } else if (d->flux == PSA_FLUX_ENGQUIST_OSHER) {
+      hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_ENGQUIST_OSHER, true, MANY>), grid, block, 0,
+                         s, a);
+    } else {
+      hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_BURGERS_UPWIND, true, MANY>), grid, block, 0,
+                         s, a);
+    }
+  } else if (d->flux == PSA_FLUX_RUSANOV) {
+    hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_RUSANOV, false, MANY>), grid, block, 0, s, a);
+  } else if (d->flux == PSA_FLUX_BURGERS_UPWIND) {
+    hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_BURGERS_UPWIND, false, MANY>), grid, block, 0,
+                       s, a);
+  } else if (d->flux == PSA_FLUX_ENGQUIST_OSHER) {
+    hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_ENGQUIST_OSHER, false, MANY>), grid, block, 0,
+                       s, a);
+  } else {
+    hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_ADVECTION_UPWIND, false, MANY>), grid, block, 0,
+                       s, a);
+  }
+}
+
+// nsub reverse steps as one launch (k_step_vjp): x, k1, k2 of the last of the
+// steps, those of the step before `stride` elements before them.
 template <typename T>
 int launch_step_vjp(const psa_solver_desc *d, const void *x, const void *k1,
                     const void *k2, const void *lam, void *out, const void *dt,
-                    hipStream_t s, long long batch = 1, int64_t ld = 0) {
+                    long long nsub, int64_t stride, hipStream_t s, long long batch,
+                    int64_t ld) {
   StepVjpArgs<T> a{};
   a.bstride = ld;
+  a.stride = stride;
+  a.nsub = static_cast<int>(nsub);
   a.v.mlp = d->mlp;
   a.v.eps4 = T(4) * static_cast<T>(d->eps);
   a.v.tau = static_cast<T>(d->mlp_tau);
@@ -1032,27 +1100,13 @@ int launch_step_vjp(const psa_solver_desc *d, const void *x, const void *k1,
   a.k2 = static_cast<const T *>(k2);
   a.lam = static_cast<const T *>(lam);
   a.out = static_cast<T *>(out);
-  const dim3 grid(static_cast<unsigned int>((d->n + kStepVjpOut - 1) / kStepVjpOut),
+  const int nout = step_vjp_out(a.nsub);
+  const dim3 grid(static_cast<unsigned int>((d->n + nout - 1) / nout),
                   static_cast<unsigned int>(batch));
-  const dim3 block(kVjpBlock);
-  if (d->mlp != nullptr) {
-    if (d->flux == PSA_FLUX_RUSANOV) {
-      hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_RUSANOV, true>), grid, block, 0, s, a);
-    } else if (d->flux == PSA_FLUX_ENGQUIST_OSHER) {
-      hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_ENGQUIST_OSHER, true>), grid, block, 0, s,
-                         a);
-    } else {
-      hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_BURGERS_UPWIND, true>), grid, block, 0, s,
-                         a);
-    }
-  } else if (d->flux == PSA_FLUX_RUSANOV) {
-    hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_RUSANOV>), grid, block, 0, s, a);
-  } else if (d->flux == PSA_FLUX_BURGERS_UPWIND) {
-    hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_BURGERS_UPWIND>), grid, block, 0, s, a);
-  } else if (d->flux == PSA_FLUX_ENGQUIST_OSHER) {
-    hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_ENGQUIST_OSHER>), grid, block, 0, s, a);
+  if (a.nsub > 1) {
+    launch_step_vjp_flux<T, true>(d, a, grid, s);
   } else {
-    hipLaunchKernelGGL((k_step_vjp<T, PSA_FLUX_ADVECTION_UPWIND>), grid, block, 0, s, a);
+    launch_step_vjp_flux<T, false>(d, a, grid, s);
   }
   return check_launch("step vjp");
 }
@@ -1235,6 +1289,25 @@ int check_batch(const psa_solver_desc *d, long long batch, long long ld) {
 // being at most the running-state array X(every)).
 bool keeps_window(long long nsteps, int every) { return nsteps > 0 && every >= nsteps; }
 
+// Whole steps the next launch takes of the `left` ones; 0 where the whole-step
+// kernels do not apply.
+long long steps_now(const psa_solver_desc *d, long long batch, long long left) {
+  const long long k = fixed_steps_per_launch(d, batch);
+  return k < left ? k : left;
+}
+
+// The step of the first checkpoint after `step`, or the last step.
+long long checkpoint_after(long long step, int every, long long nsteps) {
+  const long long next = (step / every + 1) * every;
+  return next < nsteps ? next : nsteps;
+}
+
+int batch_needs_steps() {
+  return set_error(PSA_ERR_NOT_IMPLEMENTED,
+                   "a batch runs on the whole-step kernel (default or step "
+                   "schedule, tiles 256 x 4 or 256 x 2, not Lax-Friedrichs)");
+}
+
 int forward_checkpointed(const psa_solver_desc *desc, long long batch, int64_t ld,
                          const void *u0, void *u_final, long long nsteps,
                          const void *dt, int every, void *workspace,
@@ -1256,6 +1329,7 @@ int forward_checkpointed(const psa_solver_desc *desc, long long batch, int64_t l
   char *base = static_cast<char *>(workspace);
   auto cp = [&](long long k) { return base + k * L.array_bytes; };
   char *win = cp(L.ncp);
+  const int64_t step_stride = static_cast<int64_t>(3 * L.array_bytes / elem_size(desc));
   char *cur = win + L.nwin * L.array_bytes;
   void *k1 = win, *k2 = win + L.array_bytes;
 
@@ -1269,14 +1343,16 @@ int forward_checkpointed(const psa_solver_desc *desc, long long batch, int64_t l
     auto K2 = [&](long long i) { return win + (3 * i + 2) * L.array_bytes; };
     st = copy_async(X(0), u0, bytes, s);
     if (st != PSA_OK) return st;
-    for (long long i = 0; i < nsteps; ++i) {
-      st = step_fixed_dt(desc, X(i), X(i + 1), K1(i), K2(i), dt, s, batch, ld);
-      if (st == PSA_OK) continue;
-      if (st != PSA_ERR_NOT_IMPLEMENTED) return st;
-      if (batch > 1)
-        return set_error(PSA_ERR_NOT_IMPLEMENTED,
-                         "a batch runs on the whole-step kernel (default or step "
-                         "schedule, tiles 256 x 4 or 256 x 2, not Lax-Friedrichs)");
+    for (long long i = 0; i < nsteps;) {
+      const long long k = steps_now(desc, batch, nsteps - i);
+      if (k > 0) {
+        st = steps_fixed_dt(desc, X(i), X(i + 1), K1(i), K2(i), k, step_stride, dt, s, batch,
+                            ld);
+        if (st != PSA_OK) return st;
+        i += k;
+        continue;
+      }
+      if (batch > 1) return batch_needs_steps();
       void *speed = lf_speed_slot(workspace, L);
       st = forward_stage(desc, 1, X(i), X(i), K1(i), dt, speed, s);
       if (st != PSA_OK) return st;
@@ -1284,6 +1360,7 @@ int forward_checkpointed(const psa_solver_desc *desc, long long batch, int64_t l
       if (st != PSA_OK) return st;
       st = forward_stage(desc, 3, X(i), K2(i), X(i + 1), dt, speed, s);
       if (st != PSA_OK) return st;
+      ++i;
     }
     if (nsteps % every == 0) {
       st = copy_async(cp(1), X(nsteps), bytes, s);
@@ -1296,23 +1373,23 @@ int forward_checkpointed(const psa_solver_desc *desc, long long batch, int64_t l
   // whole steps, the state alternating between cur and the window's first
   // array, where the whole-step kernel applies
   char *alt = win;
-  for (long long step = 0; step < nsteps; ++step) {
-    st = step_fixed_dt(desc, cur, alt, nullptr, nullptr, dt, s, batch, ld);
-    if (st == PSA_OK) {
+  for (long long step = 0; step < nsteps;) {
+    // (up to the next checkpoint)
+    const long long k = steps_now(desc, batch, checkpoint_after(step, every, nsteps) - step);
+    if (k > 0) {
+      st = steps_fixed_dt(desc, cur, alt, nullptr, nullptr, k, 0, dt, s, batch, ld);
+      if (st != PSA_OK) return st;
       char *tmp = cur;
       cur = alt;
       alt = tmp;
-      if ((step + 1) % every == 0) {
-        st = copy_async(cp((step + 1) / every), cur, bytes, s);
+      step += k;
+      if (step % every == 0) {
+        st = copy_async(cp(step / every), cur, bytes, s);
         if (st != PSA_OK) return st;
       }
       continue;
     }
-    if (st != PSA_ERR_NOT_IMPLEMENTED) return st;
-    if (batch > 1)
-      return set_error(PSA_ERR_NOT_IMPLEMENTED,
-                       "a batch runs on the whole-step kernel (default or step "
-                       "schedule, tiles 256 x 4 or 256 x 2, not Lax-Friedrichs)");
+    if (batch > 1) return batch_needs_steps();
     void *speed = lf_speed_slot(workspace, L);
     st = forward_stage(desc, 1, cur, cur, k1, dt, speed, s);
     if (st != PSA_OK) return st;
@@ -1320,8 +1397,9 @@ int forward_checkpointed(const psa_solver_desc *desc, long long batch, int64_t l
     if (st != PSA_OK) return st;
     st = forward_stage(desc, 3, cur, k2, cur, dt, speed, s);
     if (st != PSA_OK) return st;
-    if ((step + 1) % every == 0) {
-      st = copy_async(cp((step + 1) / every), cur, bytes, s);
+    ++step;
+    if (step % every == 0) {
+      st = copy_async(cp(step / every), cur, bytes, s);
       if (st != PSA_OK) return st;
     }
   }
@@ -1348,6 +1426,7 @@ int adjoint(const psa_solver_desc *desc, long long batch, int64_t ld, long long 
   char *base = static_cast<char *>(workspace);
   auto cp = [&](long long k) { return base + k * L.array_bytes; };
   char *win = cp(L.ncp);
+  const int64_t step_stride = static_cast<int64_t>(3 * L.array_bytes / elem_size(desc));
   auto X = [&](long long i) { return win + (3 * i) * L.array_bytes; };
   auto K1 = [&](long long i) { return win + (3 * i + 1) * L.array_bytes; };
   auto K2 = [&](long long i) { return win + (3 * i + 2) * L.array_bytes; };
@@ -1365,6 +1444,8 @@ int adjoint(const psa_solver_desc *desc, long long batch, int64_t ld, long long 
       (batch > 1 || (desc->schedule != PSA_SCHEDULE_TILE &&
                      desc->schedule != PSA_SCHEDULE_PIPELINE));
 
+  const long long reverse_most = reverse_steps_per_launch(desc, batch);
+
   st = copy_async(lam_a, lam_final, bytes, s);
   if (st != PSA_OK) return st;
   char *lam = lam_a, *lam_next = lam_b;
@@ -1379,17 +1460,19 @@ int adjoint(const psa_solver_desc *desc, long long batch, int64_t ld, long long 
       st = copy_async(X(0), cp(w), bytes, s);
       if (st != PSA_OK) return st;
     }
-    for (long long step = s0; step < s1 && !kept; ++step) {
+    for (long long step = s0; step < s1 && !kept;) {
       const long long i = step - s0;
-      // one whole step writing k1, k2 and the next state (X(every) is the
+      // whole steps writing k1, k2 and the next state (X(every) is the
       // running-state array, free in this pass)
-      st = step_fixed_dt(desc, X(i), X(i + 1), K1(i), K2(i), dt, s, batch, ld);
-      if (st == PSA_OK) continue;
-      if (st != PSA_ERR_NOT_IMPLEMENTED) return st;
-      if (batch > 1)
-        return set_error(PSA_ERR_NOT_IMPLEMENTED,
-                         "a batch runs on the whole-step kernel (default or step "
-                         "schedule, tiles 256 x 4 or 256 x 2, not Lax-Friedrichs)");
+      const long long k = steps_now(desc, batch, s1 - step);
+      if (k > 0) {
+        st = steps_fixed_dt(desc, X(i), X(i + 1), K1(i), K2(i), k, step_stride, dt, s, batch,
+                            ld);
+        if (st != PSA_OK) return st;
+        step += k;
+        continue;
+      }
+      if (batch > 1) return batch_needs_steps();
       void *speed = lf_speed_slot(workspace, L);
       st = forward_stage(desc, 1, X(i), X(i), K1(i), dt, speed, s);
       if (st != PSA_OK) return st;
@@ -1399,18 +1482,22 @@ int adjoint(const psa_solver_desc *desc, long long batch, int64_t ld, long long 
         st = forward_stage(desc, 3, X(i), K2(i), X(i + 1), dt, speed, s);
         if (st != PSA_OK) return st;
       }
+      ++step;
     }
     // reverse sweep through the window
     for (long long step = s1 - 1; step >= s0; --step) {
       const long long i = step - s0;
       if (fused_reverse) {
-        // the three reverse stages in one launch
+        // the three reverse stages of this step and of some before it in one
+        // launch
+        const long long k = reverse_most < i + 1 ? reverse_most : i + 1;
         st = desc->dtype == PSA_FLOAT64
-                 ? launch_step_vjp<double>(desc, X(i), K1(i), K2(i), lam, lam_next,
-                                           dt, s, batch, ld)
-                 : launch_step_vjp<float>(desc, X(i), K1(i), K2(i), lam, lam_next,
-                                          dt, s, batch, ld);
+                 ? launch_step_vjp<double>(desc, X(i), K1(i), K2(i), lam, lam_next, dt, k,
+                                           step_stride, s, batch, ld)
+                 : launch_step_vjp<float>(desc, X(i), K1(i), K2(i), lam, lam_next, dt, k,
+                                          step_stride, s, batch, ld);
         if (st != PSA_OK) return st;
+        step -= k - 1;
         char *tmp = lam;
         lam = lam_next;
         lam_next = tmp;

@@ -21,6 +21,7 @@
 #include "../../include/pyshocks_amd.h"
 #include "psa_internal.hpp"
 #include "stage_device.hpp"
+#include "step_host.hpp"
 #include "weno5_device.hpp"
 
 namespace psa {
@@ -721,20 +722,6 @@ struct SeqStep {
 // taken copies the state to p.out; the workgroups reduce max|u_int| of the
 // new state into step_slot[s % 3]. No launch between the steps: each one starts
 // from what the previous one left.
-// Without a control block the step is taken with the device scalar p.dt_ptr
-// (and p.k1out, p.k2out may receive the stage states).
-// Waves per SIMD the compiler keeps the registers of the FP64 WENO-JS5
-// whole-step kernels within (5: at most 96 VGPRs, which the LDS of a
-// 256-thread tile allows as well); the other variants take what they need.
-#ifndef PSA_STEP_F64_WAVES
-#define PSA_STEP_F64_WAVES 5
-#endif
-template <typename T, bool LEARNED, int REC>
-constexpr int step_min_waves() {
-  return std::is_same<T, double>::value && !LEARNED && REC == 0 ? PSA_STEP_F64_WAVES
-                                                                 : 1;
-}
-
 template <typename T, int FLUX, int VEL, int BLOCK, int CPT, bool LEARNED,
           int REC = 0>
 __global__ __attribute__((amdgpu_flat_work_group_size(1, BLOCK),
@@ -747,20 +734,6 @@ void k_step(StageArgs<T> p) {
   const int tid = threadIdx.x;
   psa_control *ctrl = p.ctrl;
   const int64_t A = static_cast<int64_t>(blockIdx.x) * SM::TO;
-
-  if (ctrl == nullptr) {
-    // a fixed step of the device scalar dt (the adjoint's forward passes);
-    // in a batch, instance blockIdx.y with its own dt
-    const int64_t off = static_cast<int64_t>(blockIdx.y) * p.bstride;
-    StageArgs<T> pb = p;
-    if (p.k1out != nullptr) pb.k1out = p.k1out + off;
-    if (p.k2out != nullptr) pb.k2out = p.k2out + off;
-    unsigned long long vmax = 0;
-    step_tile<T, FLUX, VEL, BLOCK, CPT, LEARNED, REC>(pb, A, p.dt_ptr[blockIdx.y],
-                                                      p.uk + off, p.out + off, sm, vmax,
-                                                      q, nullptr);
-    return;
-  }
 
   __shared__ T s_dt;
   __shared__ int s_go;
@@ -957,10 +930,6 @@ namespace {
 
 constexpr int kThreads = 256;
 
-inline unsigned int blocks_for(int64_t work, int per_block) {
-  return static_cast<unsigned int>((work + per_block - 1) / per_block);
-}
-
 int check_dtype(int dtype) {
   if (dtype != PSA_FLOAT64 && dtype != PSA_FLOAT32) {
     return set_error(PSA_ERR_NOT_IMPLEMENTED,
@@ -1003,17 +972,6 @@ int launch_max_abs(const T *u, int64_t m, int g, T *out,
 // --- stage dispatch ---------------------------------------------------------
 
 namespace psa {
-
-struct TileConfig {
-  int block;
-  int cpt;
-  bool pipe;  // stages 1-3: the persistent pipelined kernel
-  bool step;  // steps: the whole-step kernel where it applies
-};
-
-inline bool aligned16(const void *p) {
-  return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
-}
 
 // Workgroups the device holds at once for a kernel (CUs x occupancy),
 // queried once per kernel and device (the kernel is the template argument,
@@ -1103,12 +1061,9 @@ template <typename T, int FLUX, int VEL, int BLOCK, int CPT, bool LEARNED,
 int launch_step_cfg(const StageArgs<T> &args, hipStream_t stream) {
   constexpr int TO = StepSmem<T, BLOCK, CPT>::TO;
   StageArgs<T> a = args;
-  a.aligned = aligned16(a.uk) && aligned16(a.out) &&
-              (a.bstride * static_cast<int64_t>(sizeof(T))) % 16 == 0;
-  const unsigned int blocks = blocks_for(a.m, TO);
-  const unsigned int batch = a.batch > 1 ? static_cast<unsigned int>(a.batch) : 1u;
-  hipLaunchKernelGGL((k_step<T, FLUX, VEL, BLOCK, CPT, LEARNED, REC>), dim3(blocks, batch),
-                     dim3(BLOCK), 0, stream, a);
+  a.aligned = aligned16(a.uk) && aligned16(a.out);
+  hipLaunchKernelGGL((k_step<T, FLUX, VEL, BLOCK, CPT, LEARNED, REC>),
+                     dim3(blocks_for(a.m, TO)), dim3(BLOCK), 0, stream, a);
   return check_launch("ssprk33 step");
 }
 
@@ -1129,17 +1084,6 @@ int launch_step_tiles(const StageArgs<T> &a, TileConfig cfg,
                    "unsupported tile configuration for the whole-step kernel block=" +
                        std::to_string(cfg.block) +
                        " cells_per_thread=" + std::to_string(cfg.cpt));
-}
-
-// Whether the whole-step kernel runs the steps of this descriptor.
-inline bool step_applies(const psa_solver_desc *d, TileConfig cfg, int vel) {
-  if (!cfg.step || vel == 2 || d->nu != nullptr) return false;
-  // the stages of Lax-Friedrichs need the global max|u| of the stage before
-  if (d->flux == PSA_FLUX_LAX_FRIEDRICHS) return false;
-  if (d->flux == PSA_FLUX_ADVECTION_UPWIND && d->mlp != nullptr) return false;
-  if (cfg.block == 256 && cfg.cpt == 1)
-    return d->rec == PSA_REC_WENOJS53 && d->flux != PSA_FLUX_ESWENO;
-  return cfg.block == 256 && (cfg.cpt == 4 || cfg.cpt == 2);
 }
 
 template <typename T, int REC>
@@ -1327,11 +1271,6 @@ int launch_stage(int flux, int vel, const StageArgs<T> &a, TileConfig cfg,
                    "unsupported flux " + std::to_string(flux));
 }
 
-TileConfig default_tiles(int dtype) {
-  (void)dtype;
-  return TileConfig{256, 4, false, true};
-}
-
 int check_desc(const psa_solver_desc *d) {
   if (d == nullptr) return set_error(PSA_ERR_INVALID_ARGUMENT, "null desc");
   int st = check_dtype(d->dtype);
@@ -1389,72 +1328,6 @@ int check_desc(const psa_solver_desc *d) {
   if (d->mlp != nullptr && (!(d->mlp_tau >= 0.0) || !(d->mlp_sigma >= 0.0)))
     return set_error(PSA_ERR_INVALID_ARGUMENT, "mlp_tau and mlp_sigma must be >= 0");
   return PSA_OK;
-}
-
-TileConfig tiles_of(const psa_solver_desc *d) {
-  TileConfig c = default_tiles(d->dtype);
-  // below ~2^20 cells a grid of 1024-cell tiles leaves most of the device
-  // idle: half-size tiles double the workgroups in flight
-  if (d->n < (int64_t(1) << 20)) c.cpt = 2;
-  if (d->block > 0) c.block = d->block;
-  if (d->cells_per_thread > 0) c.cpt = d->cells_per_thread;
-  if (d->schedule == PSA_SCHEDULE_TILE) c.step = false;
-  if (d->schedule == PSA_SCHEDULE_PIPELINE) {
-    c.pipe = true;
-    c.step = false;
-  }
-  // below 2^17 cells, one cell per thread where the whole-step kernel takes
-  // it (WENO-JS5, learned weights or not): the steps there are latency, and
-  // the shorter per-thread chain makes them 8-15% shorter
-  if (d->n < (int64_t(1) << 17) && d->block <= 0 && d->cells_per_thread <= 0) {
-    TileConfig one = c;
-    one.cpt = 1;
-    const int vel =
-        d->flux != PSA_FLUX_ADVECTION_UPWIND ? 0 : (d->velocity_is_const ? 1 : 2);
-    if (step_applies(d, one, vel)) c.cpt = 1;
-  }
-  return c;
-}
-
-template <typename T>
-StageArgs<T> make_args(const psa_solver_desc *d) {
-  StageArgs<T> a{};
-  a.m = d->n + 2 * static_cast<int64_t>(d->g);
-  a.n = d->n;
-  a.g = d->g;
-  a.dx = static_cast<T>(d->dx);
-  a.inv_dx = static_cast<T>(1.0) / static_cast<T>(d->dx);
-  a.eps = static_cast<T>(d->eps);
-  a.vconst = static_cast<T>(d->velocity_const);
-  a.vel = static_cast<const T *>(d->velocity);
-  if (d->flux == PSA_FLUX_LAX_FRIEDRICHS) {
-    a.vel = nullptr;
-    a.speed = static_cast<const T *>(d->velocity);
-  }
-  a.nu = static_cast<const T *>(d->nu);
-  a.aligned = 1;
-  a.es = d->rec == PSA_REC_ESWENO32 ? 1 : 0;
-  a.rec3 = (d->rec == PSA_REC_WENOJS32 || d->rec == PSA_REC_ESWENO32) ? 1 : 0;
-  a.muscl = d->rec == PSA_REC_MUSCL ? 1 : 0;
-  a.muscls = d->rec == PSA_REC_MUSCLS ? 1 : 0;
-  a.es_delta = static_cast<T>(d->es_delta);
-  a.nowrap = d->bc == PSA_BC_GIVEN ? 1 : 0;
-  a.bcm = (d->bc == PSA_BC_NEUMANN || d->bc == PSA_BC_DIRICHLET) ? d->bc : PSA_BC_PERIODIC;
-  a.bc_l = static_cast<T>(d->bc_left);
-  a.bc_r = static_cast<T>(d->bc_right);
-  a.bc_vals = static_cast<const T *>(d->bc_values);
-  a.limiter = d->limiter;
-  a.lim_theta = static_cast<T>(d->limiter_theta);
-  a.lim_atol = static_cast<T>(d->muscl_atol);
-  a.mlp = d->mlp;
-  a.tau = static_cast<T>(d->mlp_tau);
-  a.sigma = static_cast<T>(d->mlp_sigma);
-  return a;
-}
-
-inline int vel_mode(const psa_solver_desc *d) {
-  if (d->flux != PSA_FLUX_ADVECTION_UPWIND) return 0;
-  return d->velocity_is_const ? 1 : 2;
 }
 
 template <typename T>
@@ -1547,45 +1420,6 @@ int run_steps(const psa_solver_desc *d, const void *u_in, void *u_out,
     }
   }
   return PSA_OK;
-}
-
-// One fixed-dt whole step u_in -> u_out (distinct arrays) with the device
-// scalar dt, writing the stage states into k1, k2 if they are not null, for
-// the adjoint's forward and recompute passes. Returns
-// PSA_ERR_NOT_IMPLEMENTED (and launches nothing) where the whole-step kernel
-// does not apply; the caller then runs the stage kernels.
-int step_fixed_dt(const psa_solver_desc *d, const void *u_in, void *u_out, void *k1,
-                  void *k2, const void *dt, hipStream_t stream, long long batch,
-                  int64_t ld) {
-  TileConfig cfg = tiles_of(d);
-  // a batch fills the device with its instances: there the one-cell tiles of
-  // the small single grids give way to two cells per thread (the learned
-  // step 6% faster in batches of 64, the plain one the same)
-  if (batch > 1 && cfg.cpt == 1 && d->cells_per_thread <= 0) cfg.cpt = 2;
-  const int vel = vel_mode(d);
-  if (!step_applies(d, cfg, vel)) return PSA_ERR_NOT_IMPLEMENTED;
-  if (batch < 1 || batch > 65535)
-    return set_error(PSA_ERR_INVALID_ARGUMENT, "batch must be in [1, 65535]");
-  if (d->dtype == PSA_FLOAT64) {
-    StageArgs<double> a = make_args<double>(d);
-    a.uk = a.un = static_cast<const double *>(u_in);
-    a.out = static_cast<double *>(u_out);
-    a.k1out = static_cast<double *>(k1);
-    a.k2out = static_cast<double *>(k2);
-    a.dt_ptr = static_cast<const double *>(dt);
-    a.bstride = ld;
-    a.batch = static_cast<int>(batch);
-    return launch_step<double>(d, vel, a, cfg, stream);
-  }
-  StageArgs<float> a = make_args<float>(d);
-  a.uk = a.un = static_cast<const float *>(u_in);
-  a.out = static_cast<float *>(u_out);
-  a.k1out = static_cast<float *>(k1);
-  a.k2out = static_cast<float *>(k2);
-  a.dt_ptr = static_cast<const float *>(dt);
-  a.bstride = ld;
-  a.batch = static_cast<int>(batch);
-  return launch_step<float>(d, vel, a, cfg, stream);
 }
 
 }  // namespace psa

@@ -15,13 +15,41 @@ int set_error(int code, const std::string &msg);
 // Maps a pending HIP launch error to PSA_ERR_HIP.
 int check_launch(const char *what);
 
-// One fixed-dt whole step (forward.hip): u_in -> u_out, the stage states
-// into k1, k2 if not null; PSA_ERR_NOT_IMPLEMENTED where the whole-step kernel
-// does not apply (nothing launched). A batch of instances takes one launch:
-// instance b at offset b * ld (elements) of every array, dt[b] its step.
-int step_fixed_dt(const psa_solver_desc *d, const void *u_in, void *u_out, void *k1,
-                  void *k2, const void *dt, hipStream_t stream, long long batch = 1,
-                  int64_t ld = 0);
+// Fixed-dt whole steps (fixed.hip): nsub steps from u_in in one launch, the
+// state after step s to u_out + s * stride elements (stride 0: only the last
+// one, to u_out), its stage states to k1, k2 + s * stride if not null.
+// PSA_ERR_NOT_IMPLEMENTED where the whole-step kernel does not apply (nothing
+// launched). A batch of instances takes one launch: instance b at offset
+// b * ld (elements) of every array, dt[b] its step.
+int steps_fixed_dt(const psa_solver_desc *d, const void *u_in, void *u_out, void *k1,
+                   void *k2, long long nsub, int64_t stride, const void *dt,
+                   hipStream_t stream, long long batch, int64_t ld);
+
+// Steps that a launch of steps_fixed_dt best takes (0 where it does not apply).
+int fixed_steps_per_launch(const psa_solver_desc *d, long long batch);
+
+// The steps per launch of least time for a kernel whose workgroups recompute
+// margins: launches of k steps, blocks(k) workgroups, take about
+//   fix + k (step + share * ceil(blocks(k) / 256)) microseconds,
+// fix the launch, load and drain, 256 the CUs of the device, so that more steps
+// share fix until the margins add another workgroup to every CU.
+struct StepCost {
+  double fix, step, share;
+};
+template <typename Blocks>
+int best_steps(const StepCost &c, int most, Blocks blocks) {
+  int best = 1;
+  double least = 0.0;
+  for (int k = 1; k <= most; ++k) {
+    const long long b = blocks(k);
+    const double cost = c.fix / k + c.step + c.share * static_cast<double>((b + 255) / 256);
+    if (k == 1 || cost < least) {
+      best = k;
+      least = cost;
+    }
+  }
+  return best;
+}
 
 // Limiter of the flux-limited MUSCL: a known PSA_LIMITER_*, minmod's theta
 // in [1, 2] (limiters.py:166-198), a positive slope-ratio cut-off.

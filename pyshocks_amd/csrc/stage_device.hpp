@@ -40,6 +40,36 @@ __device__ __forceinline__ T load_raw(const T *__restrict__ u, int64_t gm,
   return (gm >= 0 && gm < m) ? u[gm] : T(0);
 }
 
+// The cells first, first + 1, .. of a periodic array with n interior cells and
+// g ghosts, first >= g - n (in [g - n, g + n) but for the tiniest grids). A
+// subtraction for each index instead of a 64-bit remainder, which cost as
+// much as a reverse stage of the adjoint.
+struct PeriodicSpan {
+  int64_t lo;  // the first cell's interior index, in [0, n)
+  int64_t n;
+  int g;
+
+  __device__ __forceinline__ PeriodicSpan(int64_t first, int64_t n_, int g_)
+      : n(n_), g(g_) {
+    int64_t k = first - g_;
+    if (k < 0) {
+      k += n;
+      if (k < 0) k = k % n + n;
+    }
+    if (k >= n) k %= n;
+    lo = k;
+  }
+  template <typename T>
+  __device__ __forceinline__ T load(const T *__restrict__ u, int j) const {
+    int64_t k = lo + j;
+    if (k >= n) {
+      k -= n;
+      if (k >= n) k %= n;
+    }
+    return u[g + k];
+  }
+};
+
 // Non-negative value -> order-preserving bit pattern (NaN sorts above inf).
 __device__ __forceinline__ unsigned long long abs_bits(double v) {
   return static_cast<unsigned long long>(__double_as_longlong(fabs(v)));
@@ -162,12 +192,6 @@ struct StageArgs {
   const float *mlp;  // learned weights (LEARNED kernels)
   T tau;             // their shock threshold
   T sigma;           // their smooth threshold
-  T *k1out;          // whole-step kernel: the stage states k1, k2 as well,
-  T *k2out;          //   or null
-  int64_t bstride;   // fixed-dt whole steps of a batch: instance blockIdx.y
-                     //   at offset blockIdx.y * bstride of uk, out, k1out,
-                     //   k2out, its dt at dt_ptr[blockIdx.y]
-  int batch;         // host side: instances of the launch (grid.y)
   int step_seq;      // whole-step launch s of a controlled sequence: s mod 6
   int bcm;           // whole-step kernel: PSA_BC_PERIODIC, PSA_BC_NEUMANN or
                      //   PSA_BC_DIRICHLET (ghost cells filled by the kernel)
@@ -1090,18 +1114,18 @@ __device__ __forceinline__ void step_stage(const StageArgs<T> &p, const T *X,
 
 
 // Stores a thread's CPT values of a whole-step tile (cells j0 = 4 + CPT t ..,
-// relative to base) that fall in the output cells [12, C - 4), and with VMAX
+// relative to base) that fall in the output cells [lo, hi), and with VMAX
 // accumulates the bit pattern of max|u| of the interior ones.
 template <typename T, int BLOCK, int CPT, bool VMAX>
 __device__ __forceinline__ void step_store(const StageArgs<T> &p, int64_t base,
                                            bool fast, const T *val,
                                            T *__restrict__ dst,
-                                           unsigned long long &vmax) {
-  constexpr int C = BLOCK * CPT;
+                                           unsigned long long &vmax, int lo = 12,
+                                           int hi = BLOCK * CPT - 4) {
   constexpr int VN = Vec16<T>::n;
   const int j0 = 4 + CPT * static_cast<int>(threadIdx.x);
   const int64_t a0 = base + j0;
-  if (fast && j0 >= 12 && j0 + CPT <= C - 4) {
+  if (fast && j0 >= lo && j0 + CPT <= hi) {
     if constexpr (CPT % VN == 0) {
 #pragma unroll
       for (int r = 0; r < CPT; r += VN) {
@@ -1134,7 +1158,7 @@ __device__ __forceinline__ void step_store(const StageArgs<T> &p, int64_t base,
     for (int r = 0; r < CPT; ++r) {
       const int j = j0 + r;
       const int64_t a = a0 + r;
-      if (j >= 12 && j < C - 4 && a >= 0 && a < p.m) {
+      if (j >= lo && j < hi && a >= 0 && a < p.m) {
         dst[a] = val[r];
         if constexpr (VMAX) {
           if (a >= p.g && a < p.m - p.g) {
@@ -1174,10 +1198,8 @@ __device__ __forceinline__ void step_refill(const StageArgs<T> &p, int64_t base,
 // neighbouring tiles (16 of every C cells), with the arithmetic of the stage
 // kernels, so the results are the same bit for bit. Output cells in the ghost
 // layers are written as the periodic images they are. vmax accumulates the
-// bit pattern of max|u| of the interior cells written. With p.k1out, p.k2out
-// the stage states k1 and k2 of the output cells are written as well (they
-// are exact there). Ends with the LDS in use (a barrier before the next
-// tile).
+// bit pattern of max|u| of the interior cells written. Ends with the LDS in
+// use (a barrier before the next tile).
 //
 // Ctl supplies the step: ctl.issue() runs once the tile's loads are in
 // flight, ctl.go() and ctl.dt() are read after the workgroup's first barrier
@@ -1214,11 +1236,8 @@ __device__ __forceinline__ bool step_tile_ctl(const StageArgs<T> &p, int64_t A,
     cu.store(sm.x0, tid);
   } else if (p.bcm == PSA_BC_PERIODIC) {
     ctl.issue();
-    for (int j = tid; j < L; j += BLOCK) {
-      int64_t i = (base + j - g) % n;
-      if (i < 0) i += n;
-      sm.x0[j] = uin[g + i];
-    }
+    const PeriodicSpan span(base, n, g);
+    for (int j = tid; j < L; j += BLOCK) sm.x0[j] = span.load(uin, j);
   } else {
     ctl.issue();
     for (int j = tid; j < L; j += BLOCK) sm.x0[j] = bc_cell(p, uin, base + j);
@@ -1250,11 +1269,9 @@ __device__ __forceinline__ bool step_tile_ctl(const StageArgs<T> &p, int64_t A,
   // cells never read the cells outside [0, m), whose stage values are
   // meaningless)
   const bool refill = p.bcm != PSA_BC_PERIODIC && (base < g || base + L > m - g);
-  unsigned long long unused = 0;
   step_stage<T, FLUX, VEL, BLOCK, CPT, 1, LEARNED, REC>(p, sm.x0, sm, dt, un, val, src, q);
 #pragma unroll
   for (int r = 0; r < CPT; ++r) sm.x1[j0 + r] = val[r];
-  if (p.k1out != nullptr) step_store<T, BLOCK, CPT, false>(p, base, fast, val, p.k1out, unused);
   __syncthreads();
   if (refill) {
     step_refill<T, BLOCK, CPT>(p, base, sm.x1);
@@ -1264,7 +1281,6 @@ __device__ __forceinline__ bool step_tile_ctl(const StageArgs<T> &p, int64_t A,
   step_stage<T, FLUX, VEL, BLOCK, CPT, 2, LEARNED, REC>(p, sm.x1, sm, dt, un, val, src, q);
 #pragma unroll
   for (int r = 0; r < CPT; ++r) sm.x0[j0 + r] = val[r];
-  if (p.k2out != nullptr) step_store<T, BLOCK, CPT, false>(p, base, fast, val, p.k2out, unused);
   __syncthreads();
   if (refill) {
     step_refill<T, BLOCK, CPT>(p, base, sm.x0);
@@ -1274,6 +1290,18 @@ __device__ __forceinline__ bool step_tile_ctl(const StageArgs<T> &p, int64_t A,
 
   step_store<T, BLOCK, CPT, true>(p, base, fast, val, uout, vmax);
   return true;
+}
+
+// Waves per SIMD the compiler keeps the registers of the FP64 WENO-JS5
+// whole-step kernels within (5: at most 96 VGPRs, which the LDS of a
+// 256-thread tile allows as well); the other variants take what they need.
+#ifndef PSA_STEP_F64_WAVES
+#define PSA_STEP_F64_WAVES 5
+#endif
+template <typename T, bool LEARNED, int REC>
+constexpr int step_min_waves() {
+  return std::is_same<T, double>::value && !LEARNED && REC == 0 ? PSA_STEP_F64_WAVES
+                                                                 : 1;
 }
 
 // A step of a given dt.

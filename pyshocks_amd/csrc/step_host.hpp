@@ -1,0 +1,112 @@
+// Host-side rules shared by the launches of the fused forward kernels: tiles,
+// which schedule takes a descriptor, and the kernel arguments of a descriptor.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "../../include/pyshocks_amd.h"
+#include "psa_internal.hpp"
+#include "stage_device.hpp"
+
+namespace psa {
+
+inline unsigned int blocks_for(int64_t work, int per_block) {
+  return static_cast<unsigned int>((work + per_block - 1) / per_block);
+}
+
+struct TileConfig {
+  int block;
+  int cpt;
+  bool pipe;  // stages 1-3: the persistent pipelined kernel
+  bool step;  // steps: the whole-step kernel where it applies
+};
+
+inline bool aligned16(const void *p) {
+  return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
+}
+
+// Whether the whole-step kernel runs the steps of this descriptor.
+inline bool step_applies(const psa_solver_desc *d, TileConfig cfg, int vel) {
+  if (!cfg.step || vel == 2 || d->nu != nullptr) return false;
+  // the stages of Lax-Friedrichs need the global max|u| of the stage before
+  if (d->flux == PSA_FLUX_LAX_FRIEDRICHS) return false;
+  if (d->flux == PSA_FLUX_ADVECTION_UPWIND && d->mlp != nullptr) return false;
+  if (cfg.block == 256 && cfg.cpt == 1)
+    return d->rec == PSA_REC_WENOJS53 && d->flux != PSA_FLUX_ESWENO;
+  return cfg.block == 256 && (cfg.cpt == 4 || cfg.cpt == 2);
+}
+
+inline TileConfig default_tiles(int dtype) {
+  (void)dtype;
+  return TileConfig{256, 4, false, true};
+}
+
+inline TileConfig tiles_of(const psa_solver_desc *d) {
+  TileConfig c = default_tiles(d->dtype);
+  // below ~2^20 cells a grid of 1024-cell tiles leaves most of the device
+  // idle: half-size tiles double the workgroups in flight
+  if (d->n < (int64_t(1) << 20)) c.cpt = 2;
+  if (d->block > 0) c.block = d->block;
+  if (d->cells_per_thread > 0) c.cpt = d->cells_per_thread;
+  if (d->schedule == PSA_SCHEDULE_TILE) c.step = false;
+  if (d->schedule == PSA_SCHEDULE_PIPELINE) {
+    c.pipe = true;
+    c.step = false;
+  }
+  // below 2^17 cells, one cell per thread where the whole-step kernel takes
+  // it (WENO-JS5, learned weights or not): the steps there are latency, and
+  // the shorter per-thread chain makes them 8-15% shorter
+  if (d->n < (int64_t(1) << 17) && d->block <= 0 && d->cells_per_thread <= 0) {
+    TileConfig one = c;
+    one.cpt = 1;
+    const int vel =
+        d->flux != PSA_FLUX_ADVECTION_UPWIND ? 0 : (d->velocity_is_const ? 1 : 2);
+    if (step_applies(d, one, vel)) c.cpt = 1;
+  }
+  return c;
+}
+
+template <typename T>
+StageArgs<T> make_args(const psa_solver_desc *d) {
+  StageArgs<T> a{};
+  a.m = d->n + 2 * static_cast<int64_t>(d->g);
+  a.n = d->n;
+  a.g = d->g;
+  a.dx = static_cast<T>(d->dx);
+  a.inv_dx = static_cast<T>(1.0) / static_cast<T>(d->dx);
+  a.eps = static_cast<T>(d->eps);
+  a.vconst = static_cast<T>(d->velocity_const);
+  a.vel = static_cast<const T *>(d->velocity);
+  if (d->flux == PSA_FLUX_LAX_FRIEDRICHS) {
+    a.vel = nullptr;
+    a.speed = static_cast<const T *>(d->velocity);
+  }
+  a.nu = static_cast<const T *>(d->nu);
+  a.aligned = 1;
+  a.es = d->rec == PSA_REC_ESWENO32 ? 1 : 0;
+  a.rec3 = (d->rec == PSA_REC_WENOJS32 || d->rec == PSA_REC_ESWENO32) ? 1 : 0;
+  a.muscl = d->rec == PSA_REC_MUSCL ? 1 : 0;
+  a.muscls = d->rec == PSA_REC_MUSCLS ? 1 : 0;
+  a.es_delta = static_cast<T>(d->es_delta);
+  a.nowrap = d->bc == PSA_BC_GIVEN ? 1 : 0;
+  a.bcm = (d->bc == PSA_BC_NEUMANN || d->bc == PSA_BC_DIRICHLET) ? d->bc : PSA_BC_PERIODIC;
+  a.bc_l = static_cast<T>(d->bc_left);
+  a.bc_r = static_cast<T>(d->bc_right);
+  a.bc_vals = static_cast<const T *>(d->bc_values);
+  a.limiter = d->limiter;
+  a.lim_theta = static_cast<T>(d->limiter_theta);
+  a.lim_atol = static_cast<T>(d->muscl_atol);
+  a.mlp = d->mlp;
+  a.tau = static_cast<T>(d->mlp_tau);
+  a.sigma = static_cast<T>(d->mlp_sigma);
+  return a;
+}
+
+inline int vel_mode(const psa_solver_desc *d) {
+  if (d->flux != PSA_FLUX_ADVECTION_UPWIND) return 0;
+  return d->velocity_is_const ? 1 : 2;
+}
+
+}  // namespace psa

@@ -579,3 +579,39 @@ def test_learned_adjoint_consistency(torch_mod, kind: str) -> None:
 
 
 # }}}
+
+
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+@pytest.mark.parametrize("n,batch", [(3, 1), (8, 1), (41, 1), (237, 1), (256, 1), (2049, 1),
+                                     (61, 3), (1023, 5)])
+def test_many_steps_per_launch(torch_mod, n: int, batch: int, dtype: str) -> None:
+    """Several forward or reverse steps per launch (the numbers that the grid
+    size and the batch give, with remainders before a checkpoint and at the
+    ends; grids smaller than the margins of a tile and batches that share the
+    device) give the stage-wise kernels' states and gradients bit for bit."""
+    torch = torch_mod
+    from pyshocks_amd import _lib, burgers, make_uniform_cell_grid
+    from pyshocks_amd.adjoint import BatchedCheckpointedSolve, CheckpointedSolve
+    from pyshocks_amd.reconstruction import WENOJS53
+    from pyshocks_amd.scalar import PeriodicBoundary
+    from pyshocks_amd.timestepping import BoundOperator
+
+    dt_ = getattr(torch, dtype)
+    grid = make_uniform_cell_grid(0.0, 1.0, n, nghosts=3, dtype=dt_, device="cuda")
+    src = BoundOperator(burgers.Rusanov(rec=WENOJS53(eps=1e-6)), grid, PeriodicBoundary())
+    data = [_data(n, 40 + b) for b in range(batch)]
+    u0 = torch.tensor(np.stack([d[0] for d in data]), device="cuda").to(dt_)
+    lam = torch.tensor(np.stack([d[1] for d in data]), device="cuda").to(dt_)
+    dt = 0.2 / n
+    for nsteps, every in [(1, 1), (27, 27), (29, 14)]:
+        if batch == 1:
+            solve = CheckpointedSolve(src, u0[0].contiguous(), nsteps, dt, every=every)
+            got_u, got = solve.u_final[None], solve.gradient(lam[0])[None]
+        else:
+            bsolve = BatchedCheckpointedSolve(src, u0, nsteps, dt, every=every)
+            got_u, got = bsolve.u_final, bsolve.gradient(lam)
+        for b in range(batch):
+            ref = CheckpointedSolve(src, u0[b].contiguous(), nsteps, dt, every=every,
+                                    schedule=_lib.PSA_SCHEDULE_TILE)
+            assert torch.equal(got_u[b][3:-3], ref.u_final[3:-3]), (nsteps, b)
+            assert torch.equal(got[b], ref.gradient(lam[b].contiguous())), (nsteps, b)
