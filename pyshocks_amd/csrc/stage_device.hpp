@@ -153,6 +153,63 @@ __device__ __forceinline__ unsigned long long gather_slots(
 }
 
 // ---------------------------------------------------------------------------
+// device-side step control (timestepping.py:89-152)
+
+// Decision of stage 1, evaluated identically by every workgroup.
+__device__ __forceinline__ unsigned long long gather_umax(
+    const psa_control *ctrl) {
+  return gather_slots(ctrl->umax_slot);
+}
+
+// The fields of the control block that do not change during a call, read
+// once by the kernels that take many steps.
+template <typename T>
+struct StepParams {
+  T tfinal, theta, cfl_num, fixed_dt;
+  long long maxit;
+  int dt_mode;
+
+  __device__ __forceinline__ explicit StepParams(const psa_control *ctrl)
+      : tfinal(static_cast<T>(ctrl->tfinal)),
+        theta(static_cast<T>(ctrl->theta)),
+        cfl_num(static_cast<T>(ctrl->cfl_num)),
+        fixed_dt(static_cast<T>(ctrl->fixed_dt)),
+        maxit(ctrl->maxit),
+        dt_mode(ctrl->dt_mode) {}
+};
+
+// Whether the step from a state at time t0 after m0 steps with status
+// status0 is taken, and its dt (timestepping.py:89-152).
+template <typename T>
+__device__ __forceinline__ bool control_decide_at(const StepParams<T> &c, double t0,
+                                                  long long m0, int status0,
+                                                  unsigned long long umax_bits,
+                                                  T &dt, int &status) {
+  // (without branches: a kernel's decision runs beside its other work)
+  const T t = static_cast<T>(t0);
+  const T tfinal = c.tfinal;
+  const bool live = status0 == PSA_OK && !(t >= tfinal) && !(c.maxit >= 0 && m0 >= c.maxit);
+  const T smax = from_bits<T>(umax_bits);
+  T d = c.theta * (c.cfl_num / smax);
+  d = c.dt_mode == PSA_DT_FIXED ? c.fixed_dt : d;
+  const T dt_min = tfinal - t;
+  const T clipped = (d < dt_min ? d : dt_min) + static_cast<T>(1.0e-15);
+  d = isinf(tfinal) ? d : clipped;
+  const bool fine = isfinite(d);
+  status = live && !fine ? PSA_ERR_NONFINITE_DT : status0;
+  if (live && fine) dt = d;
+  return live && fine;
+}
+
+template <typename T>
+__device__ __forceinline__ bool control_decide(const psa_control *ctrl,
+                                               unsigned long long umax_bits,
+                                               T &dt, int &status) {
+  return control_decide_at<T>(StepParams<T>(ctrl), ctrl->t, ctrl->m, ctrl->status,
+                              umax_bits, dt, status);
+}
+
+// ---------------------------------------------------------------------------
 // fused tiled stage kernel
 
 template <typename T>

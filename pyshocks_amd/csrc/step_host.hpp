@@ -109,4 +109,21 @@ inline int vel_mode(const psa_solver_desc *d) {
   return d->velocity_is_const ? 1 : 2;
 }
 
+// Whether the ring schedule runs the steps of this descriptor (with a
+// control block): periodic, at most PSA_RING_MAX_CELLS cells, what the
+// whole-step kernel takes without learned weights.
+inline bool ring_applies(const psa_solver_desc *d, int vel) {
+  if (d->schedule != PSA_SCHEDULE_DEFAULT && d->schedule != PSA_SCHEDULE_RING) return false;
+  if (d->bc != PSA_BC_PERIODIC || d->mlp != nullptr || d->nu != nullptr || vel == 2)
+    return false;
+  if (d->flux == PSA_FLUX_LAX_FRIEDRICHS) return false;
+  return d->n >= 8 && d->n <= PSA_RING_MAX_CELLS && d->g >= 2 && d->g <= d->n;
+}
+
+// All nsteps steps of a call on the ring schedule (ring_applies), ring.hip.
+int launch_ring(const psa_solver_desc *d, const StageArgs<double> &a, long long nsteps,
+                hipStream_t stream);
+int launch_ring(const psa_solver_desc *d, const StageArgs<float> &a, long long nsteps,
+                hipStream_t stream);
+
 }  // namespace psa

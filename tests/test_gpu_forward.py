@@ -576,6 +576,29 @@ def test_ring_schedule_bit_for_bit(torch_mod, kind: str, dtype_name: str, n: int
         assert torch.equal(a[k], b[k]) and torch.equal(b[k], d[k])
 
 
+@pytest.mark.parametrize("dtype_name", ["float64", "float32"])
+@pytest.mark.parametrize("n", [46, 47, 184, 185, 440, 441, 696, 697, 880, 881])
+def test_ring_schedule_window_edges(torch_mod, dtype_name: str, n: int) -> None:
+    """Full and just-begun last windows of one, two and three cells per thread
+    and the sizes where the number changes, bit for bit against the
+    whole-step kernel."""
+    torch = torch_mod
+    from oracle import exact as E
+    from pyshocks_amd import _lib, make_uniform_cell_grid
+    from pyshocks_amd.timestepping import fused_plan
+
+    dtype = getattr(torch, dtype_name)
+    grid = make_uniform_cell_grid(0.0, 1.0, n, nghosts=3, dtype=dtype)
+    plan = fused_plan(_stepper(torch, "rusanov", grid))
+    u0 = torch.tensor(E.exact_cell_averages(E.large_initial_condition(seed=7), n),
+                      device="cuda").to(dtype)
+    a = _schedule_run(torch, plan, u0, _lib.PSA_SCHEDULE_STEP)
+    b = _schedule_run(torch, plan, u0, _lib.PSA_SCHEDULE_RING)
+    assert a[2] == b[2]
+    for k in (0, 1):
+        assert torch.equal(a[k], b[k])
+
+
 @pytest.mark.parametrize("kind", ["rusanov", "godunov", "eo", "advection"])
 @pytest.mark.parametrize("dtype_name", ["float64", "float32"])
 @pytest.mark.parametrize("n", [1500, 20000])
