@@ -773,31 +773,6 @@ int launch_max_abs(const T *u, int64_t m, int g, T *out,
 
 namespace psa {
 
-// Workgroups the device holds at once for a kernel (CUs x occupancy),
-// queried once per kernel and device (the kernel is the template argument,
-// so every kernel has a cache of its own).
-template <auto Kernel>
-unsigned int resident_blocks(int block) {
-  constexpr int kMaxDevices = 64;
-  static unsigned int cache[kMaxDevices] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
-  if (cache[dev] == 0) {
-    int per_cu = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, reinterpret_cast<const void *>(Kernel), block, 0) !=
-            hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount,
-                              dev) != hipSuccess ||
-        per_cu <= 0 || cus <= 0) {
-      (void)hipGetLastError();
-      return 0;
-    }
-    cache[dev] = static_cast<unsigned int>(per_cu) * static_cast<unsigned int>(cus);
-  }
-  return cache[dev];
-}
-
 template <typename T, int FLUX, int VEL, int STAGE, int BLOCK, int CPT,
           bool LEARNED = false, int REC = 0>
 int launch_stage_cfg(const StageArgs<T> &args, hipStream_t stream) {
@@ -1101,6 +1076,12 @@ int run_steps(const psa_solver_desc *d, const void *u_in, void *u_out,
     a.uk = un;
     a.out = uo;
     return launch_ring(d, a, nsteps, stream);
+  }
+  if (a.ctrl != nullptr && nsteps >= kMarchLeastSteps && march_applies(d, cfg, vel)) {
+    a.uk = un;
+    a.out = uo;
+    st = launch_march(d, a, nsteps, b2, stream);
+    if (st != PSA_ERR_NOT_IMPLEMENTED) return st;
   }
   if (a.ctrl != nullptr && step_applies(d, cfg, vel)) {
     // one launch per step; u^n and u^(n+1) are distinct arrays: the state

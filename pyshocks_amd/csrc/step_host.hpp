@@ -126,4 +126,53 @@ int launch_ring(const psa_solver_desc *d, const StageArgs<double> &a, long long 
 int launch_ring(const psa_solver_desc *d, const StageArgs<float> &a, long long nsteps,
                 hipStream_t stream);
 
+// Steps below which its two launches are not worth it (us a step as launches and
+// as a march, N = 16384: one step 15.4, 15.7, two 10.4, 10.8, four 7.9, 6.7), and
+// the cells that a tile's margins need.
+constexpr long long kMarchLeastSteps = 4;
+constexpr int64_t kMarchLeastCells = 64;
+
+// Whether a call's steps on this descriptor run in one launch that keeps a tile
+// per workgroup (march.hip), if the device holds its workgroups at once: the
+// default schedule and tiles of a periodic state that the whole-step kernel
+// takes, without learned weights.
+inline bool march_applies(const psa_solver_desc *d, TileConfig cfg, int vel) {
+  return d->schedule == PSA_SCHEDULE_DEFAULT && d->bc == PSA_BC_PERIODIC && d->block <= 0 &&
+         d->cells_per_thread <= 0 && d->mlp == nullptr && d->n >= kMarchLeastCells &&
+         step_applies(d, cfg, vel);
+}
+
+// The steps of a call as a march; scratch: an array of m cells of the state's
+// type. PSA_ERR_NOT_IMPLEMENTED (nothing launched) where the state is too large
+// for it or the device too small.
+int launch_march(const psa_solver_desc *d, const StageArgs<double> &a, long long nsteps,
+                 void *scratch, hipStream_t stream);
+int launch_march(const psa_solver_desc *d, const StageArgs<float> &a, long long nsteps,
+                 void *scratch, hipStream_t stream);
+
+// Workgroups the device holds at once for a kernel (CUs x occupancy),
+// queried once per kernel and device (the kernel is the template argument,
+// so every kernel has a cache of its own).
+template <auto Kernel>
+unsigned int resident_blocks(int block) {
+  constexpr int kMaxDevices = 64;
+  static unsigned int cache[kMaxDevices] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
+  if (cache[dev] == 0) {
+    int per_cu = 0, cus = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &per_cu, reinterpret_cast<const void *>(Kernel), block, 0) !=
+            hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount,
+                              dev) != hipSuccess ||
+        per_cu <= 0 || cus <= 0) {
+      (void)hipGetLastError();
+      return 0;
+    }
+    cache[dev] = static_cast<unsigned int>(per_cu) * static_cast<unsigned int>(cus);
+  }
+  return cache[dev];
+}
+
 }  // namespace psa

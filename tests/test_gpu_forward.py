@@ -629,6 +629,67 @@ def test_one_cell_per_thread_tiles_bit_for_bit(torch_mod, kind: str, dtype_name:
         assert torch.equal(r[0], runs[0][0]) and torch.equal(r[1], runs[0][1])
 
 
+@pytest.mark.parametrize("kind", ["rusanov", "godunov", "eo", "advection"])
+@pytest.mark.parametrize("dtype_name", ["float64", "float32"])
+@pytest.mark.parametrize("n", [1025, 1200, 1201, 61440, 61441, 126976, 126977, 258048, 258049])
+def test_march_bit_for_bit(torch_mod, kind: str, dtype_name: str, n: int) -> None:
+    """The steps of a call in one launch (the default schedule of mid-size
+    periodic states: full and barely more than full tiles of one, two and four
+    cells per thread, and the first size above them) compute exactly what the
+    whole-step kernel computes, over the call sequence of _schedule_run."""
+    torch = torch_mod
+    from oracle import exact as E
+    from pyshocks_amd import _lib, make_uniform_cell_grid
+    from pyshocks_amd.timestepping import fused_plan
+
+    dtype = getattr(torch, dtype_name)
+    grid = make_uniform_cell_grid(0.0, 1.0, n, nghosts=3, dtype=dtype)
+    vel = torch.ones(grid.n, dtype=dtype, device="cuda") if kind == "advection" else None
+    plan = fused_plan(_stepper(torch, kind, grid, vel=vel,
+                               theta=0.5 if kind == "advection" else 1.0))
+    u0 = torch.tensor(E.exact_cell_averages(E.large_initial_condition(seed=6), n),
+                      device="cuda").to(dtype)
+    a = _schedule_run(torch, plan, u0, _lib.PSA_SCHEDULE_STEP)
+    b = _schedule_run(torch, plan, u0, _lib.PSA_SCHEDULE_DEFAULT)
+    assert a[2] == b[2]
+    for k in (0, 1):
+        assert torch.equal(a[k], b[k])
+
+
+def test_march_in_a_graph(torch_mod) -> None:
+    """A captured call of many steps in one launch, replayed on a running
+    control block with eager work in between, continues the eager run's
+    steps bit for bit."""
+    torch = torch_mod
+    from oracle import exact as E
+    from pyshocks_amd import _lib, make_uniform_cell_grid
+    from pyshocks_amd.timestepping import fused_plan
+
+    n = 5000
+    plan = fused_plan(_stepper(torch, "rusanov", make_uniform_cell_grid(0.0, 1.0, n, nghosts=3)))
+    u0 = torch.tensor(E.exact_cell_averages(E.large_initial_condition(seed=6), n), device="cuda")
+    big = float(np.finfo(np.float64).max)
+    u, k1, k2 = u0.clone(), torch.empty_like(u0), torch.empty_like(u0)
+    ctrl = plan.new_control(u0, 0.0, big, None)
+    plan.steps(u, u, k1, k2, ctrl, 8)
+    torch.cuda.synchronize()
+    u.copy_(u0)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        plan.steps(u, u, k1, k2, ctrl, 8)
+    ctrl.copy_(plan.new_control(u0, 0.0, big, None))
+    v, kk1, kk2 = u0.clone(), torch.empty_like(u0), torch.empty_like(u0)
+    plan.desc.schedule = _lib.PSA_SCHEDULE_STEP
+    ctrl2 = plan.new_control(u0, 0.0, big, None)
+    for k in range(4):
+        graph.replay()
+        plan.steps(v, v, kk1, kk2, ctrl2, 8)
+        torch.cuda.synchronize()
+        a, b = plan.read_control(ctrl), plan.read_control(ctrl2)
+        assert (a.t, a.dt, a.m, a.status) == (b.t, b.dt, b.m, b.status) and a.m == 8 * (k + 1)
+        assert torch.equal(u, v)
+
+
 @pytest.mark.parametrize("rec", ["wenojs32", "esweno32", "muscl", "muscls", "esweno-flux"])
 @pytest.mark.parametrize("dtype_name", ["float64", "float32"])
 def test_ring_schedule_reconstructions(torch_mod, rec: str, dtype_name: str) -> None:
