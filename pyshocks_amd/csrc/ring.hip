@@ -10,110 +10,15 @@
 #include "psa_internal.hpp"
 #include "stage_device.hpp"
 #include "step_host.hpp"
+#include "wave_device.hpp"
 
 namespace psa {
 namespace {
 
 constexpr int kRingMax = PSA_RING_MAX_CELLS;
-constexpr int kRingHalo = 9;  // cells a step takes off either side of a window
 
 // Output cells of a wave's window of 64 * CPT cells.
-constexpr int ring_out(int cpt) { return 64 * cpt - 2 * kRingHalo; }
-
-// The value of the lane to the left (lane - 1; 0 in lane 0) or to the right
-// (lane + 1; 0 in lane 63): a DPP wave shift.
-template <int CTRL>
-__device__ __forceinline__ float wave_shift(float v) {
-  return __int_as_float(
-      __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
-}
-template <int CTRL>
-__device__ __forceinline__ double wave_shift(double v) {
-  return __hiloint2double(
-      __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, true),
-      __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, true));
-}
-template <typename T>
-__device__ __forceinline__ T from_left(T v) {
-  return wave_shift<0x138>(v);  // wave_shr:1
-}
-template <typename T>
-__device__ __forceinline__ T from_right(T v) {
-  return wave_shift<0x130>(v);  // wave_shl:1
-}
-
-// The flux differences of a thread's CPT cells x of the window: the stencils
-// from the neighbouring lanes, then reconstruct_any and the face fluxes of
-// step_stage (each thread the faces right of its cells, the one to its left
-// from the left lane).
-template <typename T, int FLUX, int REC, int CPT>
-__device__ __forceinline__ void ring_fluxes(const StageArgs<T> &p, const T x[CPT], T dF[CPT]) {
-  constexpr bool ES = FLUX == PSA_FLUX_ESWENO;
-  T w[CPT + 4];
-  if constexpr (CPT == 1) {
-    w[1] = from_left(x[0]);
-    w[0] = from_left(w[1]);
-    w[3] = from_right(x[0]);
-    w[4] = from_right(w[3]);
-  } else {
-    w[0] = from_left(x[CPT - 2]);
-    w[1] = from_left(x[CPT - 1]);
-    w[CPT + 2] = from_right(x[0]);
-    w[CPT + 3] = from_right(x[1]);
-  }
-#pragma unroll
-  for (int r = 0; r < CPT; ++r) w[2 + r] = x[r];
-  T ul[CPT], ur[CPT], om[ES ? CPT : 1];
-  const MlpSource src{nullptr, nullptr};
-  reconstruct_any<T, CPT, false, REC>(p, w, ul, ur, src, nullptr, 0, ES ? om : nullptr);
-  const T ulr = from_right(ul[0]);
-  T omr = T(0);
-  if constexpr (ES) omr = from_right(om[0]);
-  T F[CPT + 1];
-#pragma unroll
-  for (int k = 1; k <= CPT; ++k) {
-    const T ulR = k == CPT ? ulr : ul[k < CPT ? k : 0];
-    if constexpr (ES) {
-      F[k] = flux_burgers_upwind(ur[k - 1], ulR) +
-             es_dissipation_w(om[k - 1], k == CPT ? omr : om[k < CPT ? k : 0], w[k + 1],
-                              w[k + 2], p.es_delta);
-    } else {
-      F[k] = stage_flux<T, FLUX>(ur[k - 1], ulR, w[k + 1], w[k + 2], p.vconst);
-    }
-  }
-  F[0] = from_left(F[CPT]);
-#pragma unroll
-  for (int r = 0; r < CPT; ++r) dF[r] = F[r + 1] - F[r];
-}
-
-// Maximum of non-negative values over the wave, in lane 63 (the DPP steps of
-// wave_max_u32 on the value itself).
-template <int CTRL, int ROWS, typename T>
-__device__ __forceinline__ T dpp_max(T v) {
-  T o;
-  if constexpr (sizeof(T) == 8) {
-    o = __hiloint2double(
-        __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xF, true),
-        __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xF, true));
-  } else {
-    o = __int_as_float(
-        __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xF, true));
-  }
-  return fmax(v, o);
-}
-template <typename T>
-__device__ __forceinline__ T row_max(T v) {  // of the lane's row of 16, to all of it
-  v = dpp_max<0xB1, 0xF>(v);
-  v = dpp_max<0x4E, 0xF>(v);
-  v = dpp_max<0x124, 0xF>(v);
-  return dpp_max<0x128, 0xF>(v);
-}
-template <typename T>
-__device__ __forceinline__ T wave_max(T v) {
-  v = row_max(v);
-  v = dpp_max<0x142, 0xA>(v);
-  return dpp_max<0x143, 0xC>(v);
-}
+constexpr int ring_out(int cpt) { return 64 * cpt - 2 * kWaveHalo; }
 
 // Up to nsteps steps of the control block's sequence (the decisions of the
 // whole-step launches, control_decide_at, from the state's own max|u|); on exit
@@ -161,8 +66,8 @@ __global__ __launch_bounds__(1024) void k_ring(StageArgs<T> p, long long nsteps)
 #pragma unroll
   for (int r = 0; r < CPT; ++r) {
     const int k = CPT * lane + r;
-    const int i = wave * OUT - kRingHalo + k;
-    mine[r] = k >= kRingHalo && k < kRingHalo + OUT && i < n;
+    const int i = wave * OUT - kWaveHalo + k;
+    mine[r] = k >= kWaveHalo && k < kWaveHalo + OUT && i < n;
     int j = i % n;
     if (j < 0) j += n;
     cell[r] = j;
@@ -178,6 +83,7 @@ __global__ __launch_bounds__(1024) void k_ring(StageArgs<T> p, long long nsteps)
   bool taken = false;
   T dt_last = T(0);
   unsigned long long umax_used = umax;  // max|u| of the last decision
+  const MlpSource none{nullptr, nullptr};
   int cur = 0;
   __syncthreads();
   for (long long s = 0; s < nsteps; ++s) {
@@ -186,7 +92,7 @@ __global__ __launch_bounds__(1024) void k_ring(StageArgs<T> p, long long nsteps)
     for (int r = 0; r < CPT; ++r) u[r] = ring[cur][cell[r]];
     const T top = s_max[cur][lane & 15];
     const int top_nan = s_nan[cur];
-    ring_fluxes<T, FLUX, REC, CPT>(p, u, dF);
+    wave_fluxes<T, FLUX, false, REC, CPT>(p, u, dF, none, nullptr);
     if (s > 0 && from_state) umax = top_nan ? nan_bits<T>() : abs_bits(row_max(top));
     T dt = T(0);
     int st;
@@ -198,10 +104,10 @@ __global__ __launch_bounds__(1024) void k_ring(StageArgs<T> p, long long nsteps)
     const T lam = stage_lambda<T, FLUX>(p, dt);
 #pragma unroll
     for (int r = 0; r < CPT; ++r) x[r] = stage_value<T, 1>(u[r], u[r], lam, dF[r]);
-    ring_fluxes<T, FLUX, REC, CPT>(p, x, dF);
+    wave_fluxes<T, FLUX, false, REC, CPT>(p, x, dF, none, nullptr);
 #pragma unroll
     for (int r = 0; r < CPT; ++r) x[r] = stage_value<T, 2>(x[r], u[r], lam, dF[r]);
-    ring_fluxes<T, FLUX, REC, CPT>(p, x, dF);
+    wave_fluxes<T, FLUX, false, REC, CPT>(p, x, dF, none, nullptr);
     T mx = T(0);
     bool nan = false;
 #pragma unroll

@@ -133,13 +133,14 @@ constexpr long long kMarchLeastSteps = 4;
 constexpr int64_t kMarchLeastCells = 64;
 
 // Whether a call's steps on this descriptor run in one launch that keeps a tile
-// per workgroup (march.hip), if the device holds its workgroups at once: the
+// per workgroup (march_device.hpp), if the device holds its workgroups at once: the
 // default schedule and tiles of a periodic state that the whole-step kernel
-// takes, without learned weights.
+// takes, without learned weights, or of the Lax-Friedrichs flux.
 inline bool march_applies(const psa_solver_desc *d, TileConfig cfg, int vel) {
   return d->schedule == PSA_SCHEDULE_DEFAULT && d->bc == PSA_BC_PERIODIC && d->block <= 0 &&
          d->cells_per_thread <= 0 && d->mlp == nullptr && d->n >= kMarchLeastCells &&
-         step_applies(d, cfg, vel);
+         (step_applies(d, cfg, vel) ||
+          (d->flux == PSA_FLUX_LAX_FRIEDRICHS && d->nu == nullptr));
 }
 
 // The steps of a call as a march; scratch: an array of m cells of the state's

@@ -631,11 +631,12 @@ def test_one_cell_per_thread_tiles_bit_for_bit(torch_mod, kind: str, dtype_name:
 
 @pytest.mark.parametrize("kind", ["rusanov", "godunov", "eo", "advection"])
 @pytest.mark.parametrize("dtype_name", ["float64", "float32"])
-@pytest.mark.parametrize("n", [1025, 1200, 1201, 61440, 61441, 126976, 126977, 258048, 258049])
+@pytest.mark.parametrize("n", [1025, 1200, 47104, 47105, 112640, 112641, 243712, 243713,
+                               374784, 374785, 505856, 505857])
 def test_march_bit_for_bit(torch_mod, kind: str, dtype_name: str, n: int) -> None:
     """The steps of a call in one launch (the default schedule of mid-size
-    periodic states: full and barely more than full tiles of one, two and four
-    cells per thread, and the first size above them) compute exactly what the
+    periodic states: full and barely more than full tiles of one to eight
+    cells per lane, and the first size above them) compute exactly what the
     whole-step kernel computes, over the call sequence of _schedule_run."""
     torch = torch_mod
     from oracle import exact as E
@@ -652,6 +653,32 @@ def test_march_bit_for_bit(torch_mod, kind: str, dtype_name: str, n: int) -> Non
     a = _schedule_run(torch, plan, u0, _lib.PSA_SCHEDULE_STEP)
     b = _schedule_run(torch, plan, u0, _lib.PSA_SCHEDULE_DEFAULT)
     assert a[2] == b[2]
+    for k in (0, 1):
+        assert torch.equal(a[k], b[k])
+
+
+@pytest.mark.parametrize("dtype_name", ["float64", "float32"])
+@pytest.mark.parametrize("n", [63, 64, 184, 185, 440, 441, 952, 953, 47104, 47105, 505856,
+                               505857, 1030144, 1030145])
+def test_march_lax_friedrichs_bit_for_bit(torch_mod, dtype_name: str, n: int) -> None:
+    """Lax-Friedrichs steps of a call in one launch (one tile, several, and the
+    sizes on either side of its rule) compute exactly what the stage kernels
+    compute, over the call sequence of _schedule_run."""
+    torch = torch_mod
+    from oracle import exact as E
+    from pyshocks_amd import _lib, make_uniform_cell_grid
+    from pyshocks_amd.timestepping import fused_plan
+
+    dtype = getattr(torch, dtype_name)
+    grid = make_uniform_cell_grid(0.0, 1.0, n, nghosts=3, dtype=dtype)
+    plan = fused_plan(_stepper(torch, "lf", grid))
+    u0 = torch.tensor(E.exact_cell_averages(E.large_initial_condition(seed=6), n),
+                      device="cuda").to(dtype)
+    a = _schedule_run(torch, plan, u0, _lib.PSA_SCHEDULE_TILE)
+    b = _schedule_run(torch, plan, u0, _lib.PSA_SCHEDULE_DEFAULT)
+    # (t, dt, m and the start's max|u| of each control block; the march leaves the
+    # final state's maximum combined, the stage kernels leave partials of it)
+    assert [f[:4] for f in a[2]] == [f[:4] for f in b[2]]
     for k in (0, 1):
         assert torch.equal(a[k], b[k])
 
