@@ -381,11 +381,15 @@ typedef struct psa_solver_desc {
  *   block, tiles 256 x 4 or 256 x 2). Steps ping-pong between u_out and the
  *   stage buffers.
  * RING: one launch for all the steps of the call; one workgroup holds a
- *   periodic state of n <= PSA_RING_MAX_CELLS cells in LDS (one cell per
- *   thread) and takes the steps with the arithmetic and the decisions of
+ *   periodic state of n <= PSA_RING_MAX_CELLS cells in its waves' registers
+ *   and takes the steps with the arithmetic and the decisions of
  *   STEP, with no HBM traffic between steps (what STEP takes, periodic, no
  *   learned weights; the stage buffers are not used).
- * DEFAULT is RING where it applies, else STEP where it applies, else TILE.
+ * DEFAULT is RING where it applies, else, for calls of at least 4 steps on a
+ *   mid-size periodic state without learned weights or Rusanov nu (up to
+ *   505856 cells; MUSCL 243712; Lax-Friedrichs in FP32 1030144; default tiles),
+ *   one launch whose workgroups hold a tile each and exchange edges and
+ *   maxima through k2, else STEP where it applies, else TILE.
  * All schedules compute the same values. */
 #define PSA_SCHEDULE_DEFAULT 0
 #define PSA_SCHEDULE_TILE 1
@@ -419,6 +423,12 @@ int psa_control_init(const psa_solver_desc *desc, const void *u,
 int psa_ssprk33_steps(const psa_solver_desc *desc, const void *u_in,
                       void *u_out, void *k1, void *k2, void *control,
                       long long nsteps, void *stream);
+
+/* 1 if a psa_ssprk33_steps call of 4 or more steps on this descriptor (with a
+ * valid control block) runs them all in one launch, which ends with the last
+ * step that is taken, so that enqueuing more steps than a run needs costs
+ * nothing; 0 if not. */
+int psa_ssprk33_one_launch(const psa_solver_desc *desc);
 
 /* One stage (1, 2 or 3) of timestepping.py:312-320: stage 1 out = uk + dt L(uk),
  * stage 2 out = 3/4 un + 1/4 (uk + dt L(uk)), stage 3 out = 1/3 un +

@@ -210,6 +210,7 @@ SIGNATURES: dict[str, list[Any]] = {
     "psa_numerical_flux_desc": [ctypes.POINTER(PsaSolverDesc), _VP, _VP, _VP, _VP],
     "psa_ssprk33_steps": [ctypes.POINTER(PsaSolverDesc), _VP, _VP, _VP, _VP,
                           _VP, _LL, _VP],
+    "psa_ssprk33_one_launch": [ctypes.POINTER(PsaSolverDesc)],
     "psa_ssprk33_advance": [ctypes.POINTER(PsaSolverDesc), _VP, _VP, _VP, _VP,
                             _VP, _VP],
     "psa_ssprk33_stage": [ctypes.POINTER(PsaSolverDesc), _I, _VP, _VP, _VP, _VP,

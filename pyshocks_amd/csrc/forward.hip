@@ -354,7 +354,15 @@ __global__ void k_control_init(psa_control *ctrl, double t, double tfinal,
                                double theta, double cfl_num, double fixed_dt,
                                long long maxit, int dt_mode,
                                int speed_from_state, double speed_const) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  // (a lane per slot)
+  static_assert(PSA_UMAX_SLOTS == 64, "one wave");
+  const int k = static_cast<int>(threadIdx.x);
+  const unsigned long long bits = abs_bits(static_cast<T>(speed_const));
+  ctrl->umax_slot[k][0] = k == 0 ? bits : 0ull;
+  ctrl->speed_slot[0][k][0] = 0ull;
+  ctrl->speed_slot[1][k][0] = 0ull;
+  for (int b = 0; b < 3; ++b) ctrl->step_slot[b][k][0] = 0ull;
+  if (k != 0) return;
   ctrl->t = t;
   ctrl->dt = 0.0;
   ctrl->tfinal = tfinal;
@@ -363,14 +371,7 @@ __global__ void k_control_init(psa_control *ctrl, double t, double tfinal,
   ctrl->fixed_dt = fixed_dt;
   ctrl->m = 0;
   ctrl->maxit = maxit;
-  ctrl->umax_bits = abs_bits(static_cast<T>(speed_const));
-  for (int k = 0; k < PSA_UMAX_SLOTS; ++k) {
-    ctrl->umax_slot[k][0] = 0ull;
-    ctrl->speed_slot[0][k][0] = 0ull;
-    ctrl->speed_slot[1][k][0] = 0ull;
-    for (int b = 0; b < 3; ++b) ctrl->step_slot[b][k][0] = 0ull;
-  }
-  ctrl->umax_slot[0][0] = ctrl->umax_bits;
+  ctrl->umax_bits = bits;
   for (int b = 0; b < 2; ++b) {
     ctrl->seq_t[b] = t;
     ctrl->seq_m[b] = 0;
@@ -1750,6 +1751,17 @@ int psa_ssprk33_steps(const psa_solver_desc *desc, const void *u_in,
                              nsteps, s);
   return run_steps<float>(desc, u_in, u_out, k1, k2, control, nullptr, nsteps,
                           s);
+}
+
+int psa_ssprk33_one_launch(const psa_solver_desc *desc) {
+  if (check_desc(desc) != PSA_OK) return 0;
+  const int vel = vel_mode(desc);
+  if (ring_applies(desc, vel)) return 1;
+  if (!march_applies(desc, tiles_of(desc), vel)) return 0;
+  const int st = desc->dtype == PSA_FLOAT64
+                     ? launch_march(desc, make_args<double>(desc), 0, nullptr, nullptr)
+                     : launch_march(desc, make_args<float>(desc), 0, nullptr, nullptr);
+  return st == PSA_OK ? 1 : 0;
 }
 
 int psa_ssprk33_stage(const psa_solver_desc *desc, int stage, const void *un,

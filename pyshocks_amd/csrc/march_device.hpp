@@ -174,8 +174,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
   const MlpSource none{nullptr, nullptr};
   __syncthreads();
 
-  // The maximum of |x| over the own cells of all waves; with a tag, also the
-  // neighbour tiles' edge cells of that step into the outer slots. False: the
+  // The maximum of |x| over the own cells of all waves; with s_edge, also the
+  // neighbour tiles' edge cells of the step of the tag into its outer slots. False: the
   // wait was given up. Every thread of the launch takes part.
   auto exchange = [&](unsigned long long tag, T (*s_edge)[2][kHalo],
                       unsigned long long &top) -> bool {
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     // tiles a wave)
     const long long began = wall_clock64();
     bool ok = true;
-    if (tag != 0 && wave == kWaves - 1) {
+    if (s_edge != nullptr && wave == kWaves - 1) {
       const bool mine = lane < 2 * X::SIDE;
       const int side = lane < X::SIDE ? 0 : 1;
       const int k = lane - side * X::SIDE;
@@ -410,12 +410,14 @@ int launch_march_cells(const StageArgs<T> &a, MarchArgs<T> f, void *scratch, hip
   const unsigned int resident = resident_blocks<k_march<T, FLUX, REC, CPT>>(kBlock);
   if (resident < 4u * static_cast<unsigned int>(tiles)) return PSA_ERR_NOT_IMPLEMENTED;
   // the exchange words and the abort flag in the caller's scratch array
+  // (no scratch: the caller asks whether it would run)
   const uintptr_t at =
       (reinterpret_cast<uintptr_t>(scratch) + 127u) & ~static_cast<uintptr_t>(127);
   const int count = tiles > 1 ? Exchange<T>::count(tiles) : 0;
   const size_t need = sizeof(unsigned long long) * static_cast<size_t>(count) + sizeof(int) +
                       (at - reinterpret_cast<uintptr_t>(scratch));
   if (need > static_cast<size_t>(a.m) * sizeof(T)) return PSA_ERR_NOT_IMPLEMENTED;
+  if (scratch == nullptr) return PSA_OK;
   f.x.words = reinterpret_cast<unsigned long long *>(at);
   f.x.tiles = tiles;
   f.abort = reinterpret_cast<int *>(f.x.words + count);

@@ -145,7 +145,8 @@ inline bool march_applies(const psa_solver_desc *d, TileConfig cfg, int vel) {
 
 // The steps of a call as a march; scratch: an array of m cells of the state's
 // type. PSA_ERR_NOT_IMPLEMENTED (nothing launched) where the state is too large
-// for it or the device too small.
+// for it or the device too small. With a null scratch: the same answer, and
+// nothing is launched.
 int launch_march(const psa_solver_desc *d, const StageArgs<double> &a, long long nsteps,
                  void *scratch, hipStream_t stream);
 int launch_march(const psa_solver_desc *d, const StageArgs<float> &a, long long nsteps,
