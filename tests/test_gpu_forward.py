@@ -657,6 +657,70 @@ def test_march_bit_for_bit(torch_mod, kind: str, dtype_name: str, n: int) -> Non
         assert torch.equal(a[k], b[k])
 
 
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 6, 511, 512, 513, 1024, 4099])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_reconstruct_pair_edges(torch_mod, n: int, offset: int) -> None:
+    """The two-cell FP64 reconstruction at the ends of the array, of its
+    workgroups and on arrays that are not 16-byte aligned, and nothing written
+    beside them. Six indicators, products and the reciprocal leave some 20
+    roundings in a weight and the candidates are at most 10/3 max|f|, twice (the
+    oracle rounds too): 2 * 20 * 10/3 * 2^-53 max|f| at most, of which the sums'
+    cancellation shows a tenth."""
+    torch = torch_mod
+    from oracle import weno_np as W
+    from pyshocks_amd import _lib
+
+    rng = np.random.default_rng(n)
+    f = rng.standard_normal(n) + np.where(np.arange(n) % 7 < 3, 2.0, 0.0)
+    if n > 8:
+        f[n // 2] = 1.0e70  # indicators past the shared reciprocal's range
+        f[3] = np.nan
+    buf = torch.zeros(n + 1, dtype=torch.float64, device="cuda")
+    buf[offset:offset + n] = torch.tensor(f)
+    out = torch.full((2, n + 3), 9.0, dtype=torch.float64, device="cuda")
+    ul, ur = (out[k, offset:offset + n] for k in (0, 1))
+    x = buf[offset:offset + n]
+    _lib.call("psa_reconstruct", _lib.PSA_FLOAT64, _lib.PSA_REC_WENOJS53, _lib.ptr(x),
+              _lib.ptr(ul), _lib.ptr(ur), n, 1e-6, _lib.stream_of(x))
+    pad = np.concatenate([np.zeros(2), f, np.zeros(2)])
+    scale = np.nanmax(np.abs([pad[k:k + n] for k in range(5)]), axis=0)
+    with np.errstate(all="ignore"):
+        ref = W.reconstruct(pad, 1e-6, "wenojs53")  # (zeros outside the array)
+    for got, want in zip((ul, ur), ref):
+        got, want = got.cpu().numpy(), want[2:-2]
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        ok = np.isnan(want) | (np.abs(got - want) <= 1.5e-14 * scale)
+        assert ok.all()
+    out[0, offset:offset + n] = 9.0
+    out[1, offset:offset + n] = 9.0
+    assert (out == 9.0).all()
+
+
+@pytest.mark.parametrize("dtype_name", ["float64", "float32"])
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 4095, 4097, 1 << 21, (1 << 21) + 5])
+def test_max_abs_edges(torch_mod, dtype_name: str, n: int) -> None:
+    """max|u| of the interior with its largest value at either end, in the
+    unaligned first and last cells, and NaN above all; the ghost cells (larger)
+    stay out."""
+    torch = torch_mod
+    from pyshocks_amd.reductions import max_abs_interior
+
+    dtype = getattr(torch, dtype_name)
+    for off in range(4):
+        for g in (0, 3):
+            buf = torch.full((n + 2 * g + off,), 100.0, dtype=dtype, device="cuda")
+            u = buf[off:]
+            v = u[g:g + n]
+            v.copy_(torch.linspace(-1.0, 0.5, n, dtype=dtype, device="cuda"))
+            for at in {0, 1, n // 2, n - 2, n - 1} & set(range(n)):
+                old = v[at].clone()
+                v[at] = -3.0
+                assert max_abs_interior(u, g).item() == 3.0
+                v[at] = float("nan")
+                assert np.isnan(max_abs_interior(u, g).item())
+                v[at] = old
+
+
 @pytest.mark.parametrize("dtype_name", ["float64", "float32"])
 @pytest.mark.parametrize("n", [63, 64, 184, 185, 440, 441, 952, 953, 47104, 47105, 505856,
                                505857, 1030144, 1030145])
