@@ -490,8 +490,8 @@ typedef struct psa_batch_desc {
                                    (FP32 states then end exactly at tfinal) */
   int max_team;                 /* largest team size (teams only)          */
   /* Teams (all NULL/0: one workgroup per instance, in `order`). Instance i
-   * is advanced by team[i] workgroups that split its tiles and meet at a
-   * device-wide barrier after every stage; the queue is then the nslots
+   * is advanced by team[i] workgroups that split its tiles and meet after
+   * every step (PSA_SCHEDULE_TILE: every stage); the queue is then the nslots
    * slots (slot_inst[s], slot_rank[s]) listing each instance's members
    * consecutively, ranks 0 .. team[i] - 1. team_state is caller-owned device
    * scratch of ninst * PSA_TEAM_STATE_BYTES bytes, cleared by the call.
@@ -505,9 +505,10 @@ typedef struct psa_batch_desc {
   void *team_state;
   double team_wait_s;
   /* PSA_SCHEDULE_STEP (or DEFAULT): one pass per step over an instance's
-   * tiles with the three stages of a tile in LDS (step_tile of the
-   * whole-step kernel; one barrier per step, the state ping-pongs between
-   * u and k1); PSA_SCHEDULE_TILE: one pass and one barrier per stage. Both
+   * tiles with the three stages of a tile in a wave's registers (the state
+   * ping-pongs between u and k1; the members of a team exchange edge cells
+   * and maxima through k2, and one without room for its words there stays
+   * out); PSA_SCHEDULE_TILE: one pass and one barrier per stage. Both
    * compute the same values. PSA_FLUX_LAX_FRIEDRICHS (WENO-JS5 weights,
    * no learned weights) always takes the stage passes: each stage's flux
    * speed is max|u| of its input over the instance, reduced after the

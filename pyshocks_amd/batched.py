@@ -196,8 +196,9 @@ class BatchedSolver:
                    wait_s: float) -> None:
         """Instances above ``team_cells`` cells (``None``: the work rule of
         :meth:`_work_teams`) are split among a team of ``ceil(m / team_cells)``
-        workgroups (at most ``max_team``, at most one per tile) that meet at a
-        device-wide barrier after every stage."""
+        workgroups (at most ``max_team``, at most one per tile) that exchange
+        edge cells and maxima after every step (schedule "tile": meet at a
+        device-wide barrier after every stage)."""
         tile = (self.desc.block or 256) * (self.desc.cells_per_thread or 4)
         ntiles = (self.m + tile - 1) // tile
         cap = np.minimum(max_team, ntiles)

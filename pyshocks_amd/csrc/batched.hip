@@ -4,15 +4,16 @@
 // Work is a queue of slots (an atomic counter over a caller-provided list,
 // longest instances first). A slot is one member of an instance's team: an
 // instance of team size 1 is run by one workgroup alone, a large instance by
-// a team of workgroups that split its tiles and meet at a global barrier
-// after every stage. Every member runs the instance's whole time loop: the
+// a team of workgroups that split its cells and meet after every step (stage
+// sweeps: at a global barrier after every stage). Every member runs the instance's whole time loop: the
 // CFL time step of timestepping.py:89-152 with predict_timestep of
 // burgers/schemes.py:42-49,121-127 (Rusanov with alpha = 1 or Godunov), and
 // the three SSP-RK3 stages of timestepping.py:312-320, each a sweep over its
-// tiles with the same tile computation as the single-instance stage kernels.
+// tiles with the same tile computation as the single-instance stage kernels,
+// or the step as one sweep of wave tiles (the default schedule).
 // max|u| of each new state is reduced in the workgroup and, for a team,
-// through an atomic in the team's state block; all members take the same dt
-// from the same reduced value, so they stop at the same step.
+// through an atomic in the team's state block or exchange words; all members
+// take the same dt from the same reduced value, so they stop at the same step.
 //
 // Termination: the grid never exceeds the workgroups the device holds at
 // once, and teams never exceed the grid, so every slot is eventually taken
@@ -30,8 +31,10 @@
 #include <type_traits>
 
 #include "../../include/pyshocks_amd.h"
+#include "exchange_device.hpp"
 #include "psa_internal.hpp"
 #include "stage_device.hpp"
+#include "wave_device.hpp"
 
 namespace psa {
 namespace {
@@ -41,14 +44,13 @@ struct TeamState {
   unsigned int arrive;  // barrier arrivals, monotone
   int abort;
   unsigned int pad0[2];
-  // max|u| bits: stage sweeps alternate between the first two (cleared
-  // after the first barrier of a step); whole-step sweeps rotate over all
-  // three (one barrier per step)
-  unsigned long long umax[3];
+  // max|u| bits: stage sweeps alternate between the two (cleared after the
+  // first barrier of a step)
+  unsigned long long umax[2];
   // Lax-Friedrichs: max|k1| and max|k2| of the step, the flux speeds of
   // stages 2 and 3 (each cleared after the barrier that follows its reads)
   unsigned long long speed[2];
-  unsigned long long pad1[1];
+  unsigned long long pad1[2];
 };
 static_assert(sizeof(TeamState) == PSA_TEAM_STATE_BYTES, "team state size");
 
@@ -104,6 +106,14 @@ __device__ __forceinline__ unsigned long long wave_uniform(unsigned long long v)
   return (static_cast<unsigned long long>(hi) << 32) | lo;
 }
 
+__device__ __forceinline__ float wave_uniform(float v) {
+  return __int_as_float(wave_uniform(__float_as_int(v)));
+}
+__device__ __forceinline__ double wave_uniform(double v) {
+  return __longlong_as_double(static_cast<long long>(
+      wave_uniform(static_cast<unsigned long long>(__double_as_longlong(v)))));
+}
+
 template <int BLOCK>
 __device__ __forceinline__ unsigned long long block_max_bcast(
     unsigned long long v, unsigned long long *s_red,
@@ -153,22 +163,103 @@ __device__ __forceinline__ bool team_barrier(TeamState *ts, int size,
   return wave_uniform(*s_flag) != 0;
 }
 
-// WHOLE: one sweep per step with the three stages of each tile in LDS
-// (step_tile), the state alternating between u and k1; otherwise one sweep
-// per stage (stage_tile).
+// Cells per lane of the wave tiles of the whole-step sweep: as many as the
+// registers hold beside the loop's (4096 instances of 128 to 65536 cells, FP32:
+// 4 cells 108 ms, 8 cells 103; FP64: 4 cells 149, 6 cells 145).
+template <typename T, int CPT, bool LEARNED>
+constexpr int batch_cells() {
+  return LEARNED ? 4 : sizeof(T) == 4 ? 2 * CPT : CPT + 2;
+}
+
+// Waves per SIMD that the registers leave room for.
+template <typename T, bool LEARNED, bool WHOLE, int BLOCK>
+constexpr int batch_min_waves() {
+  return WHOLE && !LEARNED && (BLOCK > 512 || sizeof(T) == 4) ? 4
+         : WHOLE && !LEARNED                                  ? 3
+                                                              : (BLOCK + 255) / 256;
+}
+
+// LDS of the whole-step sweep: the waves' maxima (two sets, used in turn, for
+// the waves of a single workgroup meet once a step), the team's, and the cells
+// beside this member's.
+template <typename T, int WAVES>
+struct TeamSmem {
+  unsigned long long red[2][WAVES];
+  unsigned long long top;
+  T halo[2][kWaveHalo];
+  int abort;
+};
+
+// Members that advance an instance: as many as its team has and as its k2 array
+// holds exchange words for (each then owns more cells than a halo).
+template <typename T>
+__device__ __forceinline__ int team_members(int size, int64_t m) {
+  const int64_t most = m * static_cast<int64_t>(sizeof(T)) /
+                       (Exchange<T>::count(1) * static_cast<int64_t>(sizeof(long long)));
+  return size <= most ? size : (most > 1 ? static_cast<int>(most) : 1);
+}
+
+// First interior cell of member r of `size`: the array's cells from there on are
+// 16-byte aligned.
+__device__ __forceinline__ int64_t member_begin(int64_t n, int g, int r, int size) {
+  if (r == 0) return 0;
+  if (r == size) return n;
+  return ((n * r / size + g) & ~static_cast<int64_t>(3)) - g;
+}
+
+// The exchange words of all teams as no step waits for them.
+template <typename T>
+__global__ __launch_bounds__(64) void k_batch_words(BatchArgs<T> a) {
+  for (long long k = blockIdx.x; k < a.nslots; k += gridDim.x) {
+    const int i = a.order[k];
+    const int64_t m = a.ncells[i] + 2 * static_cast<int64_t>(a.g);
+    const int size = team_members<T>(a.team[i], m);
+    const int rank = a.slot_rank[k];
+    if (size < 2 || rank >= size) continue;
+    const Exchange<T> x{reinterpret_cast<unsigned long long *>(a.k2 + a.offsets[i]), size};
+    const int tid = threadIdx.x;
+    if (tid < 2) *x.max_word(tid, rank) = kTurn;
+    for (int w = tid; w < 4 * Exchange<T>::SIDE; w += 64)
+      x.cells(w / (2 * Exchange<T>::SIDE), rank, w / Exchange<T>::SIDE % 2)
+          [w % Exchange<T>::SIDE] = 0ull;
+  }
+}
+
+// WHOLE: one sweep per step, the state alternating between u and k1, a wave
+// tile (wave_step) per wave at a time; otherwise one sweep per stage
+// (stage_tile).
 // REC: the reconstruction class of the fused kernels (0 WENO-JS5 or learned,
 // 1 third order, 2 MUSCL, 3 slope-limited MUSCL).
+//
+// WHOLE: the members of a team own a range of interior cells each, read and
+// written by themselves only; what they need of each other, nine cells on
+// either side and the maximum, goes through exchange words (in the instance's
+// k2 array), so that a step needs no write-back or invalidation of an L2, which
+// holds the states of every other workgroup of the XCD too. With fences at every
+// step and a tile per workgroup in LDS the same batches took, ms before and
+// after (default tiles): 1024 instances of 128 to 65536 cells FP32 60.0, 27.5,
+// FP64 67.8, 38.1; 512 of 1024 to 16384 29.8, 7.1 and 28.8, 8.3; 64 of 4096 to
+// 65536 FP32 28.9, 10.8; 256 of 1024 to 32768 with learned weights FP64 25.9,
+// 18.3; 4096 of 128 to 65536 FP32 113, 103 (bound by the FP32 rate: 174e9 cell
+// updates a second of some 195e9 that the whole-step arithmetic allows), FP64
+// 179, 145.
 template <typename T, int FLUX, int BLOCK, int CPT, bool LEARNED, bool WHOLE, int REC>
-__global__ __launch_bounds__(BLOCK) void k_batch(BatchArgs<T> a) {
-  using Smem = typename std::conditional<WHOLE,
-                                         StepSmem<T, BLOCK, CPT, FLUX == PSA_FLUX_ESWENO>,
+__global__ __launch_bounds__(BLOCK)
+    __attribute__((amdgpu_waves_per_eu((batch_min_waves<T, LEARNED, WHOLE, BLOCK>()))))
+void k_batch(BatchArgs<T> a) {
+  constexpr int WAVES = BLOCK / 64;
+  constexpr int WCPT = batch_cells<T, CPT, LEARNED>();
+  constexpr int TILE = BLOCK * CPT;  // of the stage sweeps
+  using Smem = typename std::conditional<WHOLE, TeamSmem<T, WAVES>,
                                          StageSmem<T, 0, BLOCK, CPT>>::type;
-  constexpr int TILE = WHOLE ? StepSmem<T, BLOCK, CPT>::TO : BLOCK * CPT;
   __shared__ Smem sm;
   __shared__ unsigned long long s_bcast;
   __shared__ long long s_next;
   __shared__ int s_flag;
-  __shared__ unsigned int q[LEARNED ? (BLOCK / 64) * learned_queue_words<CPT>() : 1];
+  constexpr int QW = LEARNED ? (WHOLE ? learned_queue_words<WCPT>()
+                                      : learned_queue_words<CPT>())
+                             : 0;
+  __shared__ unsigned int q[LEARNED ? WAVES * QW : 1];
   const int tid = threadIdx.x;
   // a persistent workgroup keeps the network's operand registers in LDS
   __shared__ MlpLdsSlot<LEARNED> wl;
@@ -191,15 +282,19 @@ __global__ __launch_bounds__(BLOCK) void k_batch(BatchArgs<T> a) {
     if (k >= a.nslots) break;
     const int i = a.order[k];
     const int rank = a.slot_rank != nullptr ? a.slot_rank[k] : 0;
-    const int size = a.team != nullptr ? a.team[i] : 1;
+    int size = a.team != nullptr ? a.team[i] : 1;
+    if constexpr (WHOLE) {
+      size = team_members<T>(size, a.ncells[i] + 2 * static_cast<int64_t>(a.g));
+      if (rank >= size) continue;
+    }
     TeamState *ts = size > 1 ? a.teams + i : nullptr;
 
     StageArgs<T> p{};
     p.n = a.ncells[i];
     p.g = a.g;
     p.m = p.n + 2 * static_cast<int64_t>(a.g);
-    p.dx = static_cast<T>(a.dx[i]);
-    p.inv_dx = T(1) / p.dx;
+    p.dx = wave_uniform(static_cast<T>(a.dx[i]));
+    p.inv_dx = wave_uniform(T(1) / p.dx);
     p.eps = a.eps;
     p.mlp = a.mlp;
     p.tau = a.tau;
@@ -212,29 +307,122 @@ __global__ __launch_bounds__(BLOCK) void k_batch(BatchArgs<T> a) {
     T *u = a.u + a.offsets[i];
     T *k1 = a.k1 + a.offsets[i];
     T *k2 = a.k2 + a.offsets[i];
+    bool alive = true;
+
+    // ---- WHOLE: this member's interior cells [own_lo, own_hi), the exchange
+    const int64_t own_lo = member_begin(p.n, p.g, rank, size);
+    const int64_t own_hi = member_begin(p.n, p.g, rank + 1, size);
+    [[maybe_unused]] const Exchange<T> ex{reinterpret_cast<unsigned long long *>(k2), size};
+    [[maybe_unused]] unsigned int turns = 0;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // The maximum of v over the instance; with a tag, also the neighbours' edge
+    // cells of that step (into sm.halo).
+    [[maybe_unused]] auto exchange = [&](unsigned long long v,
+                                         unsigned long long tag) -> unsigned long long {
+      using X = Exchange<T>;
+      const int set = static_cast<int>(turns & 1u);
+      const unsigned long long turn = (turns & 2u) != 0 ? kTurn : 0ull;
+      ++turns;
+      if constexpr (WHOLE) {
+        v = wave_max_u64(v);
+        if ((tid & 63) == 0) sm.red[set][wave] = v;
+        __syncthreads();
+        v = sm.red[set][0];
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) v = sm.red[set][w] > v ? sm.red[set][w] : v;
+        if (ts == nullptr) return wave_uniform(v);
+        const int lane = tid & 63;
+        if (tid == 0) put(ex.max_word(set, rank), turn | v);
+        // wave 0 waits for every member's maximum, the last wave for the
+        // neighbours' edges
+        const long long began = wall_clock64();
+        bool ok = true;
+        auto waits = [&](unsigned int spin) {
+          if (spin % 32 != 1) return true;
+          return wall_clock64() - began <= a.wait_ticks &&
+                 __hip_atomic_load(&ts->abort, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT) == 0;
+        };
+        if (tag != 0 && wave == WAVES - 1) {
+          const bool mine = lane < 2 * X::SIDE;
+          const int side = lane < X::SIDE ? 0 : 1;
+          const int k = lane - side * X::SIDE;
+          const int left = rank == 0 ? size - 1 : rank - 1;
+          const int right = rank == size - 1 ? 0 : rank + 1;
+          const unsigned long long *w =
+              ex.cells(set, side == 0 ? left : right, side == 0 ? 1 : 0) + (mine ? k : 0);
+          unsigned long long c = tag;
+          for (unsigned int spin = 1; ok; ++spin) {
+            if (mine) c = get(w);
+            if (__all((c & 0xFFFFFFFF00000000ull) == tag)) break;
+            ok = waits(spin);
+          }
+          const unsigned int bits = static_cast<unsigned int>(c);
+          if constexpr (X::NW == 2) {
+            const unsigned int hi = __shfl_down(bits, 1, 64);
+            if (mine && (k & 1) == 0)
+              sm.halo[side][k >> 1] =
+                  __hiloint2double(static_cast<int>(hi), static_cast<int>(bits));
+          } else {
+            if (mine) sm.halo[side][k] = __uint_as_float(bits);
+          }
+          if (!ok && lane == 0) sm.abort = 1;
+        }
+        if (wave == 0) {
+          unsigned long long most = 0;
+          for (int r0 = 0; r0 < size; r0 += 64) {
+            const bool mine = r0 + lane < size;
+            const unsigned long long *w = ex.max_word(set, mine ? r0 + lane : 0);
+            unsigned long long c = turn;
+            for (unsigned int spin = 1; ok; ++spin) {
+              if (mine) c = get(w);
+              if (__all((c & kTurn) == turn)) break;
+              ok = waits(spin);
+            }
+            const unsigned long long v2 = wave_max_u64(mine ? c & ~kTurn : 0ull);
+            most = v2 > most ? v2 : most;
+          }
+          if (lane == 0) {
+            sm.top = most;
+            if (!ok) sm.abort = 1;
+          }
+        }
+        __syncthreads();
+        if (sm.abort != 0) {
+          alive = false;
+          if (tid == 0)
+            __hip_atomic_store(&ts->abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        v = sm.top;
+      }
+      return wave_uniform(v);
+    };
+
+    // ---- stage sweeps: tiles of the array, barriers through the team state
     const int64_t ntiles = (p.m + TILE - 1) / TILE;
     // this member's tiles
     const int64_t tlo = ntiles * rank / size;
     const int64_t thi = ntiles * (rank + 1) / size;
     unsigned int nbar = 0;
-    bool alive = true;
 
     // team reduction of max|u| bits into buffer b (a single workgroup keeps
     // the block maximum)
-    // (b = 0 .. 2: umax[b]; 3, 4: speed[b - 3])
-    auto team_max = [&](unsigned long long v, int b) -> unsigned long long {
-      v = wave_uniform(block_max_bcast<BLOCK>(v, sm.red, &s_bcast));
-      if (ts == nullptr) return v;
-      unsigned long long *slot = b < 3 ? &ts->umax[b] : &ts->speed[b - 3];
-      if (tid == 0 && v != 0)
-        __hip_atomic_fetch_max(slot, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      alive = alive && team_barrier(ts, size, ++nbar, a.wait_ticks, &s_flag);
-      if (tid == 0)
-        s_bcast = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __syncthreads();
+    // (b = 0, 1: umax[b]; 2, 3: speed[b - 2])
+    [[maybe_unused]] auto team_max = [&](unsigned long long v, int b) -> unsigned long long {
+      if constexpr (!WHOLE) {
+        v = wave_uniform(block_max_bcast<BLOCK>(v, sm.red, &s_bcast));
+        if (ts == nullptr) return v;
+        unsigned long long *slot = b < 2 ? &ts->umax[b] : &ts->speed[b - 2];
+        if (tid == 0 && v != 0)
+          __hip_atomic_fetch_max(slot, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        alive = alive && team_barrier(ts, size, ++nbar, a.wait_ticks, &s_flag);
+        if (tid == 0)
+          s_bcast = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+      }
       return wave_uniform(s_bcast);
     };
-    auto barrier = [&]() {
+    [[maybe_unused]] auto barrier = [&]() {
       if (ts == nullptr) {
         __syncthreads();
       } else {
@@ -245,23 +433,43 @@ __global__ __launch_bounds__(BLOCK) void k_batch(BatchArgs<T> a) {
     // max |u_int| of the initial state over this member's cells
     unsigned long long vb = 0;
     {
-      int64_t lo = tlo * TILE, hi = thi * TILE;
-      lo = lo > a.g ? lo : a.g;
-      hi = hi < p.m - a.g ? hi : p.m - a.g;
+      int64_t lo, hi;
+      if constexpr (WHOLE) {
+        lo = a.g + own_lo;
+        hi = a.g + own_hi;
+      } else {
+        lo = tlo * TILE;
+        hi = thi * TILE;
+        lo = lo > a.g ? lo : a.g;
+        hi = hi < p.m - a.g ? hi : p.m - a.g;
+      }
       for (int64_t j = lo + tid; j < hi; j += BLOCK) {
         const unsigned long long b = abs_bits(u[j]);
         vb = b > vb ? b : vb;
       }
     }
-    unsigned long long umax = team_max(vb, WHOLE ? 2 : 1);
+    unsigned long long umax;
+    if constexpr (WHOLE) {
+      if (ts != nullptr && tid < 2 * kWaveHalo) {
+        // the initial cells beside this member's
+        const int side = tid < kWaveHalo ? 0 : 1;
+        const int k = tid - side * kWaveHalo;
+        const PeriodicSpan span((side == 0 ? own_lo - kWaveHalo : own_hi) + p.g, p.n, p.g);
+        sm.halo[side][k] = span.load(u, k);
+      }
+      if (tid == 0) sm.abort = 0;
+      umax = exchange(vb, 0ull);
+    } else {
+      umax = team_max(vb, 1);
+    }
 
     // time control: in the state dtype (timestepping.py:136-152), or with
     // time_f64 in FP64 (t and the unclipped dt; the stages use dt rounded to
     // the state dtype and t advances by exactly that value)
-    const double tf64 = a.tfinal[i];
-    const double cfl64 = 0.5 * a.dx[i];  // 0.5 dx^(2 - alpha), alpha = 1
-    const T tf = static_cast<T>(tf64);
-    const T cfl = T(0.5) * p.dx;
+    const double tf64 = wave_uniform(a.tfinal[i]);
+    const double cfl64 = wave_uniform(0.5 * a.dx[i]);  // 0.5 dx^(2 - alpha), alpha = 1
+    const T tf = wave_uniform(static_cast<T>(tf64));
+    const T cfl = wave_uniform(T(0.5) * p.dx);
     T t = T(0);
     double t64 = 0.0;
     long long steps = 0;
@@ -308,21 +516,79 @@ __global__ __launch_bounds__(BLOCK) void k_batch(BatchArgs<T> a) {
         }
       }
 
+      dt = wave_uniform(dt);
+      dt_t64 = wave_uniform(dt_t64);
       if constexpr (WHOLE) {
-        // every member has read the max|u| of two steps ago (before the
-        // barrier of the previous step): clear it for the next step
-        if (ts != nullptr && rank == 0 && tid == 0)
-          __hip_atomic_store(&ts->umax[(steps + 1) % 3], 0ull, __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT);
+        using W = WaveTile<T, WCPT>;
+        using X = Exchange<T>;
         const T *src = (steps & 1) ? k1 : u;
         T *dst = (steps & 1) ? u : k1;
+        const MlpSource net{p.mlp, wlp};
+        const unsigned long long tag =
+            static_cast<unsigned long long>(static_cast<unsigned int>(steps + 1)) << 32;
+        const int set = static_cast<int>(turns & 1u);
         unsigned long long vmax = 0;
-        for (int64_t tile = tlo; tile < thi; ++tile) {
-          __syncthreads();
-          step_tile<T, FLUX, 0, BLOCK, CPT, LEARNED, REC>(p, tile * TILE, dt, src, dst,
-                                                          sm, vmax, q, wlp);
+        // the member's cells in the array, tiles from a 16-byte boundary on
+        const int64_t lo = p.g + own_lo, hi = p.g + own_hi;
+        const int64_t first = lo & ~static_cast<int64_t>(3);
+        const int64_t count = (hi - first + W::OUT - 1) / W::OUT;
+        for (int64_t tile = wave; tile < count; tile += WAVES) {
+          const int64_t base = first + tile * W::OUT - W::LO;
+          const bool inside = base >= lo && base + W::C <= hi;
+          T x[WCPT];
+          if (inside) {
+            wave_load<T, WCPT>(src, base, x);
+          } else if (ts == nullptr) {
+            // (the instance's other end)
+            const int k0 = wave_cell0<WCPT>();
+            const PeriodicSpan span(base, p.n, p.g);
+#pragma unroll
+            for (int r = 0; r < WCPT; ++r) x[r] = span.load(src, k0 + r);
+          } else {
+            const int k0 = wave_cell0<WCPT>();
+#pragma unroll
+            for (int r = 0; r < WCPT; ++r) {
+              const int64_t c = base + k0 + r;
+              // (cells further out reach no cell that is kept)
+              if (c < lo) {
+                const int64_t k = c - (lo - kWaveHalo);
+                x[r] = sm.halo[0][k > 0 ? k : 0];
+              } else if (c >= hi) {
+                const int64_t k = c - hi;
+                x[r] = sm.halo[1][k < kWaveHalo ? k : kWaveHalo - 1];
+              } else {
+                x[r] = src[c];
+              }
+            }
+          }
+          wave_step<T, FLUX, LEARNED, REC, WCPT>(p, x, dt, net, q);
+          if (inside) {
+            const unsigned long long v = wave_store<T, WCPT>(dst, base, x);
+            vmax = v > vmax ? v : vmax;
+            continue;
+          }
+          const int k0 = wave_cell0<WCPT>();
+#pragma unroll
+          for (int r = 0; r < WCPT; ++r) {
+            const int64_t c = base + k0 + r;
+            if (k0 + r < W::LO || k0 + r >= W::C - W::LO || c < lo || c >= hi) continue;
+            dst[c] = x[r];
+            const unsigned long long v = abs_bits(x[r]);
+            vmax = v > vmax ? v : vmax;
+            if (ts != nullptr) {
+#pragma unroll
+              for (int k = 0; k < X::NW; ++k) {
+                if (c < lo + kWaveHalo)
+                  put(ex.cells(set, rank, 0) + X::NW * (c - lo) + k,
+                      tag | word_of(x[r], k));
+                if (c >= hi - kWaveHalo)
+                  put(ex.cells(set, rank, 1) + X::NW * (c - (hi - kWaveHalo)) + k,
+                      tag | word_of(x[r], k));
+              }
+            }
+          }
         }
-        umax = team_max(vmax, static_cast<int>(steps % 3));  // u^(n+1) complete
+        umax = exchange(vmax, tag);
       } else {
         // Lax-Friedrichs (scalar.py:276-277): the flux speed of each stage is
         // max|u| of its input over the instance (its ghosts are images of
@@ -340,7 +606,7 @@ __global__ __launch_bounds__(BLOCK) void k_batch(BatchArgs<T> a) {
               p, tile * TILE, dt, sm, v1, q, wlp);
         }
         if constexpr (kLF) {
-          p.vconst = from_bits<T>(team_max(v1, 3));  // k1 complete
+          p.vconst = from_bits<T>(team_max(v1, 2));  // k1 complete
         } else {
           barrier();  // k1 complete
         }
@@ -357,7 +623,7 @@ __global__ __launch_bounds__(BLOCK) void k_batch(BatchArgs<T> a) {
               p, tile * TILE, dt, sm, v2, q, wlp);
         }
         if constexpr (kLF) {
-          p.vconst = from_bits<T>(team_max(v2, 4));  // k2 complete
+          p.vconst = from_bits<T>(team_max(v2, 3));  // k2 complete
           // every member has read max|k1| (after the barrier before this
           // one); the next writes come after the step's last barrier
           if (ts != nullptr && rank == 0 && tid == 0)
@@ -383,17 +649,19 @@ __global__ __launch_bounds__(BLOCK) void k_batch(BatchArgs<T> a) {
                                __HIP_MEMORY_SCOPE_AGENT);
         }
       }
-      t = t + dt;
-      t64 = t64 + dt_t64;
+      t = wave_uniform(t + dt);
+      t64 = wave_uniform(t64 + dt_t64);
       steps += 1;
     }
     if (!alive) status = PSA_ERR_HIP;
     if constexpr (WHOLE) {
-      if (steps & 1) {
-        // the last state is in k1: this member's cells back to u
-        int64_t lo = tlo * TILE, hi = thi * TILE;
-        hi = hi < p.m ? hi : p.m;
-        for (int64_t j = lo + tid; j < hi; j += BLOCK) u[j] = k1[j];
+      // the last state to u where it is in k1, and its ghost cells
+      const T *last = (steps & 1) ? k1 : u;
+      for (int64_t j = own_lo + tid; j < own_hi && steps > 0; j += BLOCK) {
+        const T v = last[p.g + j];
+        if (steps & 1) u[p.g + j] = v;
+        if (j < p.g) u[p.g + p.n + j] = v;
+        if (j >= p.n - p.g) u[p.g + j - p.n] = v;
       }
     }
     if (tid == 0 && rank == 0) {
@@ -415,7 +683,6 @@ __global__ void k_batch_reset(unsigned int *counter, TeamState *teams,
     teams[j].abort = 0;
     teams[j].umax[0] = 0ull;
     teams[j].umax[1] = 0ull;
-    teams[j].umax[2] = 0ull;
     teams[j].speed[0] = 0ull;
     teams[j].speed[1] = 0ull;
   }
@@ -479,6 +746,12 @@ int launch_batch_cfg(const BatchArgs<T> &a, int grid, int max_team, long long nt
   hipLaunchKernelGGL(k_batch_reset, dim3(rb), dim3(256), 0, s, a.counter, a.teams, nt);
   int st = check_launch("batch reset");
   if (st != PSA_OK) return st;
+  if (WHOLE && max_team > 1) {
+    const unsigned int wb = a.nslots < 4096 ? static_cast<unsigned int>(a.nslots) : 4096u;
+    hipLaunchKernelGGL(k_batch_words<T>, dim3(wb), dim3(64), 0, s, a);
+    st = check_launch("batch exchange words");
+    if (st != PSA_OK) return st;
+  }
   hipLaunchKernelGGL((k_batch<T, FLUX, BLOCK, CPT, LEARNED, WHOLE, REC>), dim3(blocks),
                      dim3(BLOCK), 0, s, a);
   return check_launch("batch solve");

@@ -32,7 +32,7 @@ struct FixedArgs {
 };
 
 // nsub steps of the tile of blockIdx.x: the workgroup holds C + 8 cells of the
-// state (step_tile's layout) and computes C of them in every stage; each step
+// state (step_tile_ctl's layout) and computes C of them in every stage; each step
 // takes 9 exact cells off either side (step_tile_ctl), so after nsub of them
 // the cells [11 + 9 (nsub - 1), C - 3 - 9 (nsub - 1)) are exact and the output
 // cells lie inside. The neighbouring tiles recompute the margins; the results

@@ -648,7 +648,7 @@ __global__ __launch_bounds__(BLOCK) void k_stage_pipe(StageArgs<T> p) {
 }
 
 // ---------------------------------------------------------------------------
-// whole-step kernel (step_tile): the three SSP-RK3 stages of a tile in LDS
+// whole-step kernel (step_tile_ctl): the three SSP-RK3 stages of a tile in LDS
 
 // Before the first whole-step launch of a psa_ssprk33_steps call (one wave):
 // the state's t, m and status into entry 0 of the sequence record, max|u|

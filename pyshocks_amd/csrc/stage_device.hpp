@@ -1361,27 +1361,4 @@ constexpr int step_min_waves() {
                                                                  : 1;
 }
 
-// A step of a given dt.
-template <typename T>
-struct FixedStep {
-  T v;
-  __device__ __forceinline__ void issue() const {}
-  __device__ __forceinline__ bool go() const { return true; }
-  __device__ __forceinline__ T dt() const { return v; }
-};
-
-template <typename T, int FLUX, int VEL, int BLOCK, int CPT, bool LEARNED,
-          int REC = 0>
-__device__ __forceinline__ void step_tile(const StageArgs<T> &p, int64_t A, T dt,
-                                          const T *__restrict__ uin,
-                                          T *__restrict__ uout,
-                                          StepSmem<T, BLOCK, CPT,
-                                                   FLUX == PSA_FLUX_ESWENO> &sm,
-                                          unsigned long long &vmax,
-                                          unsigned int *q,
-                                          const MlpWaveLds *wl) {
-  step_tile_ctl<T, FLUX, VEL, BLOCK, CPT, LEARNED, REC>(p, A, FixedStep<T>{dt}, uin, uout,
-                                                        sm, vmax, q, wl);
-}
-
 }  // namespace psa

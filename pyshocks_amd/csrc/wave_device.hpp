@@ -111,7 +111,7 @@ __device__ __forceinline__ T wave_max(T v) {
   return dpp_max<0x143, 0xC>(v);
 }
 
-// Output cells of a tile are the cells [lo, 64 CPT - lo), lo a multiple of the
+// Output cells of a tile are the cells [LO, 64 CPT - LO), LO a multiple of the
 // 16-byte vectors, so that the tiles of an aligned array load and store whole
 // vectors.
 template <typename T, int CPT>
@@ -122,125 +122,71 @@ struct WaveTile {
   static_assert(LO >= kWaveHalo, "exact output cells");
 };
 
-// Cells base + CPT lane + r of the state u: 16-byte loads for a tile in the
-// interior of an aligned array, else cell by cell with the ghost fill.
-template <typename T, int CPT>
-__device__ __forceinline__ void wave_load(const StageArgs<T> &p, const T *__restrict__ u,
-                                          int64_t base, bool fast, T x[CPT]) {
-  constexpr int VN = Vec16<T>::n;
-  const int k0 = CPT * static_cast<int>(threadIdx.x & 63);
-  if (fast) {
-    const T *s = u + base + k0;
-    if constexpr (CPT % VN == 0) {
-#pragma unroll
-      for (int r = 0; r < CPT; r += VN) {
-        const typename Vec16<T>::type v = load16(s + r);
-        x[r] = v.x;
-        x[r + 1] = v.y;
-        if constexpr (VN == 4) {
-          x[r + 2] = v.z;
-          x[r + 3] = v.w;
-        }
-      }
-    } else {
-#pragma unroll
-      for (int r = 0; r < CPT; ++r) x[r] = s[r];
-    }
-  } else if (p.bcm == PSA_BC_PERIODIC) {
-    const PeriodicSpan span(base, p.n, p.g);
-#pragma unroll
-    for (int r = 0; r < CPT; ++r) x[r] = span.load(u, k0 + r);
-  } else {
-#pragma unroll
-    for (int r = 0; r < CPT; ++r) x[r] = bc_cell(p, u, base + k0 + r);
-  }
+// The lane's first cell in the tile, opaque to the compiler: the masks that come
+// from it are made where they are used, not kept in registers over the tiles of
+// a loop.
+template <int CPT>
+__device__ __forceinline__ int wave_cell0() {
+  int k0 = CPT * static_cast<int>(threadIdx.x & 63);
+  asm volatile("" : "+v"(k0));
+  return k0;
 }
 
-// The tile's output cells to u (as load: whole vectors in the interior).
+// Cells base + CPT lane + r of the array u, all of it readable, base a multiple
+// of the 16-byte vectors.
 template <typename T, int CPT>
-__device__ __forceinline__ void wave_store(const StageArgs<T> &p, T *__restrict__ u,
-                                           int64_t base, bool fast, const T x[CPT]) {
-  using W = WaveTile<T, CPT>;
+__device__ __forceinline__ void wave_load(const T *__restrict__ u, int64_t base, T x[CPT]) {
   constexpr int VN = Vec16<T>::n;
-  const int k0 = CPT * static_cast<int>(threadIdx.x & 63);
-  if (fast) {
-    T *d = u + base + k0;
-    if constexpr (CPT % VN == 0) {
+  static_assert(CPT % VN == 0, "whole vectors");
+  const T *s = u + base + wave_cell0<CPT>();
 #pragma unroll
-      for (int r = 0; r < CPT; r += VN) {
-        typename Vec16<T>::type v;
-        if constexpr (VN == 2) {
-          v = {x[r], x[r + 1]};
-        } else {
-          v = {x[r], x[r + 1], x[r + 2], x[r + 3]};
-        }
-        if (k0 + r >= W::LO && k0 + r < W::C - W::LO) store16(d + r, v);
-      }
-    } else {
-#pragma unroll
-      for (int r = 0; r < CPT; ++r)
-        if (k0 + r >= W::LO && k0 + r < W::C - W::LO) d[r] = x[r];
-    }
-  } else {
-#pragma unroll
-    for (int r = 0; r < CPT; ++r) {
-      const int k = k0 + r;
-      const int64_t a = base + k;
-      if (k >= W::LO && k < W::C - W::LO && a >= 0 && a < p.m) u[a] = x[r];
+  for (int r = 0; r < CPT; r += VN) {
+    const typename Vec16<T>::type v = load16(s + r);
+    x[r] = v.x;
+    x[r + 1] = v.y;
+    if constexpr (VN == 4) {
+      x[r + 2] = v.z;
+      x[r + 3] = v.w;
     }
   }
 }
 
-// Bit pattern of max|u| of the tile's output cells that are interior cells (the
-// NaN pattern if one is NaN).
+// The tile's output cells to u, and the bit pattern of their max|u| (the NaN
+// pattern if one is NaN).
 template <typename T, int CPT>
-__device__ __forceinline__ unsigned long long wave_max_cells(const StageArgs<T> &p,
-                                                             int64_t base, bool fast,
-                                                             const T x[CPT]) {
+__device__ __forceinline__ unsigned long long wave_store(T *__restrict__ u, int64_t base,
+                                                         const T x[CPT]) {
   using W = WaveTile<T, CPT>;
-  const int k0 = CPT * static_cast<int>(threadIdx.x & 63);
+  constexpr int VN = Vec16<T>::n;
+  const int k0 = wave_cell0<CPT>();
+  T *d = u + base + k0;
   T mx = T(0);
   bool nan = false;
 #pragma unroll
-  for (int r = 0; r < CPT; ++r) {
-    const int k = k0 + r;
-    const int64_t a = base + k;
-    const bool out = k >= W::LO && k < W::C - W::LO && (fast || (a >= p.g && a < p.m - p.g));
-    mx = fmax(mx, out ? fabs(x[r]) : T(0));
-    nan |= out && isnan(x[r]);
+  for (int r = 0; r < CPT; r += VN) {
+    typename Vec16<T>::type v;
+    if constexpr (VN == 2) {
+      v = {x[r], x[r + 1]};
+    } else {
+      v = {x[r], x[r + 1], x[r + 2], x[r + 3]};
+    }
+    const bool out = k0 + r >= W::LO && k0 + r < W::C - W::LO;
+    if (out) store16(d + r, v);
+#pragma unroll
+    for (int k = r; k < r + VN; ++k) {
+      mx = fmax(mx, out ? fabs(x[k]) : T(0));
+      nan |= out && isnan(x[k]);
+    }
   }
   return nan ? nan_bits<T>() : abs_bits(mx);
 }
 
-// The ghost cells of a non-periodic boundary in a stage's output, from its
-// interior cells (bc_cell): through the wave's LDS buffer.
-template <typename T, int CPT>
-__device__ __forceinline__ void wave_refill(const StageArgs<T> &p, int64_t base, T x[CPT],
-                                            T *buf) {
-  const int k0 = CPT * static_cast<int>(threadIdx.x & 63);
-  __builtin_amdgcn_wave_barrier();
-#pragma unroll
-  for (int r = 0; r < CPT; ++r) buf[k0 + r] = x[r];
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-  for (int r = 0; r < CPT; ++r) {
-    const int64_t a = base + k0 + r;
-    if ((a >= 0 && a < p.g) || (a >= p.m - p.g && a < p.m)) x[r] = bc_cell(p, buf - base, a);
-  }
-}
-
 // One SSP-RK3 step (timestepping.py:312-320) of the tile: u is u^n on entry and
 // u^(n+1) on return, exact on all but the 9 outermost cells of either side, the
-// bits of the stage kernels. refill: the tile holds ghost cells of a
-// non-periodic boundary, which each stage's output gets back before the next
-// stage reads it (buf).
+// bits of the stage kernels.
 template <typename T, int FLUX, bool LEARNED, int REC, int CPT>
 __device__ __forceinline__ void wave_step(const StageArgs<T> &p, T u[CPT], T dt,
-                                          const MlpSource &src, unsigned int *q,
-                                          bool refill = false, int64_t base = 0,
-                                          T *buf = nullptr) {
+                                          const MlpSource &src, unsigned int *q) {
   const T lam = stage_lambda<T, FLUX>(p, dt);
   T x[CPT];
 #pragma unroll
@@ -261,7 +207,6 @@ __device__ __forceinline__ void wave_step(const StageArgs<T> &p, T u[CPT], T dt,
 #pragma unroll
       for (int r = 0; r < CPT; ++r) x[r] = stage_value<T, 3>(x[r], u[r], lam, dF[r]);
     }
-    if (refill && stage < 3) wave_refill<T, CPT>(p, base, x, buf);
   }
 #pragma unroll
   for (int r = 0; r < CPT; ++r) u[r] = x[r];

@@ -289,3 +289,42 @@ def test_kernel_info_and_autotune_skip_spills(torch_mod) -> None:
         assert BatchedSolver(ns, dtype=dtype, tiles=best).kernel_info()["private_bytes"] == 0
         for cand in times:
             assert BatchedSolver(ns, dtype=dtype, tiles=cand).kernel_info()["private_bytes"] == 0
+
+
+@pytest.mark.parametrize("dtype_name", ["float64", "float32"])
+@pytest.mark.parametrize("tiles,g", [((256, 4), 3), ((256, 2), 5), ((1024, 2), 3)])
+def test_team_members_edges(torch_mod, dtype_name: str, tiles, g: int) -> None:
+    """The members of a team own ranges of cells and exchange nine on either
+    side: teams of seven, also on instances too small for seven, whose array
+    holds exchange words for fewer, and one workgroup per instance compute what
+    the stage sweeps compute, ghost cells included, bit for bit; sizes around a
+    wave tile, a member's least cells and a halo."""
+    torch = torch_mod
+    from pyshocks_amd.batched import BatchedSolver
+
+    class Sevens(BatchedSolver):
+        def _work_teams(self, cap):
+            return np.full(self.ninst, 7, dtype=np.int32)
+
+    dtype = getattr(torch, dtype_name)
+    ns = np.array([g, 8, 9, 10, 18, 19, 153, 154, 236, 237, 282, 283, 320, 364, 365, 488,
+                   489, 700, 1117, 1118, 2000, 3416, 4099, 7000])
+    runs = []
+    for make, kw in ((BatchedSolver, {"team_cells": 0, "schedule": "tile"}),
+                     (BatchedSolver, {"team_cells": 0}), (Sevens, {})):
+        s = make(ns, dtype=dtype, eps=1e-6, tiles=tiles, nghosts=g, **kw)
+        states = []
+        for i, n in enumerate(ns):
+            x = (np.arange(n) + 0.5) / n
+            u = 0.4 + np.sin(2 * np.pi * (x + 0.1 * i)) + 0.5 * (x > 0.6)
+            states.append(np.concatenate([u[n - g:], u, u[:g]]))
+        s.set_states(states)
+        print("solve", dtype_name, tiles, kw, int(s.team.max()), flush=True)
+        r = s.solve([min(0.05, 30.5 * 0.5 / n / 2.0) for n in ns])
+        assert (r.status == 0).all()
+        runs.append((r.t, r.steps, [s.state(i).cpu() for i in range(len(ns))]))
+    for other in runs[1:]:
+        assert np.array_equal(runs[0][0], other[0])
+        assert np.array_equal(runs[0][1], other[1])
+        for a, b in zip(runs[0][2], other[2]):
+            assert torch.equal(a, b)
