@@ -22,6 +22,7 @@
 #include "psa_internal.hpp"
 #include "stage_device.hpp"
 #include "step_host.hpp"
+#include "wave_device.hpp"
 #include "weno5_device.hpp"
 
 namespace psa {
@@ -776,6 +777,66 @@ void k_step(StageArgs<T> p) {
   }
 }
 
+// The same on wave tiles: a wave computes its tile in registers, with no LDS and
+// no barrier but the one behind the decision (periodic states, WENO-JS5). Bound
+// by the FP64 instruction rate; us a step with LDS tiles and with wave tiles of 6
+// cells per lane: N = 2^21 22.5, 21.2; 2^22 39.3, 38.0; 2^24 135.4, 126.5 (8 cells
+// per lane 127.2).
+template <typename T, int FLUX, int VEL, int CPT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_step_wave(
+    StageArgs<T> p) {
+  using W = WaveTile<T, CPT>;
+  constexpr int WAVES = 4;
+  __shared__ unsigned long long s_red[WAVES];
+  __shared__ T s_dt;
+  __shared__ int s_go;
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  psa_control *ctrl = p.ctrl;
+  const int64_t tile = static_cast<int64_t>(blockIdx.x) * WAVES + wave;
+  // outputs are the cells of the array [base + LO, base + C - LO)
+  const int64_t base = tile * W::OUT - W::LO;
+  const bool inside = p.aligned && base >= p.g && base + W::C <= p.m - p.g;
+  T x[CPT];
+  if (inside) {
+    wave_load<T, CPT>(p.uk, base, x);
+  } else {
+    const int k0 = wave_cell0<CPT>();
+    const PeriodicSpan span(base, p.n, p.g);
+#pragma unroll
+    for (int r = 0; r < CPT; ++r) x[r] = span.load(p.uk, k0 + r);
+  }
+  const SeqStep<T> ctl{ctrl, p.step_seq, &s_dt, &s_go};
+  ctl.issue();
+  __syncthreads();
+  const bool go = ctl.go();
+  unsigned long long vmax = 0;
+  if (go) {
+    const MlpSource none{nullptr, nullptr};
+    wave_step<T, FLUX, false, 0, CPT>(p, x, ctl.dt(), none, nullptr);
+  }
+  if (inside) {
+    vmax = wave_store<T, CPT>(p.out, base, x);
+  } else {
+    const int k0 = wave_cell0<CPT>();
+#pragma unroll
+    for (int r = 0; r < CPT; ++r) {
+      const int k = k0 + r;
+      const int64_t c = base + k;
+      if (k < W::LO || k >= W::C - W::LO || c >= p.m) continue;
+      // (a step not taken: the ghost cells as given)
+      p.out[c] = go ? x[r] : p.uk[c];
+      const unsigned long long v = abs_bits(x[r]);
+      if (c >= p.g && c < p.m - p.g) vmax = v > vmax ? v : vmax;
+    }
+  }
+  if (go && ctrl->speed_from_state != 0) {
+    vmax = block_max_bits<256>(vmax, s_red);
+    if (tid == 0)
+      atomicMax(&ctrl->step_slot[p.step_seq % 3][blockIdx.x % PSA_UMAX_SLOTS][0], vmax);
+  }
+}
+
 template <typename T>
 __global__ void k_copy(const T *__restrict__ src, T *__restrict__ dst,
                        int64_t m) {
@@ -942,9 +1003,41 @@ int launch_step_rec(const psa_solver_desc *d, const StageArgs<T> &a, TileConfig 
   return launch_step_tiles<T, PSA_FLUX_ADVECTION_UPWIND, 1, false, REC>(a, cfg, stream);
 }
 
+// Whether the steps of a call that the whole-step kernel takes run on wave
+// tiles: the default schedule and tiles of a large periodic WENO-JS5 state in
+// FP64 without learned weights. Below 2^21 cells the wider tiles' last wave of
+// workgroups costs as much as they save (N = 1500001: 17.1 us as LDS tiles, 18.4);
+// in FP32 the LDS tiles are faster (N = 2^24: 86.4 us, 90.1).
+inline bool step_wave_applies(const psa_solver_desc *d) {
+  return d->dtype == PSA_FLOAT64 && d->schedule == PSA_SCHEDULE_DEFAULT && d->block <= 0 &&
+         d->cells_per_thread <= 0 && d->bc == PSA_BC_PERIODIC && d->mlp == nullptr &&
+         d->rec == PSA_REC_WENOJS53 && d->n >= (int64_t(1) << 21);
+}
+
+template <int FLUX, int VEL>
+int launch_step_wave(const StageArgs<double> &args, hipStream_t stream) {
+  constexpr int CPT = 6;
+  StageArgs<double> a = args;
+  a.aligned = aligned16(a.uk) && aligned16(a.out);
+  hipLaunchKernelGGL((k_step_wave<double, FLUX, VEL, CPT>),
+                     dim3(blocks_for(a.m, 4 * WaveTile<double, CPT>::OUT)), dim3(256), 0,
+                     stream, a);
+  return check_launch("ssprk33 step (wave tiles)");
+}
+
 template <typename T>
 int launch_step(const psa_solver_desc *d, int vel, const StageArgs<T> &a,
                 TileConfig cfg, hipStream_t stream) {
+  if constexpr (std::is_same<T, double>::value) {
+    if (step_wave_applies(d)) {
+      if (d->flux == PSA_FLUX_RUSANOV) return launch_step_wave<PSA_FLUX_RUSANOV, 0>(a, stream);
+      if (d->flux == PSA_FLUX_BURGERS_UPWIND)
+        return launch_step_wave<PSA_FLUX_BURGERS_UPWIND, 0>(a, stream);
+      if (d->flux == PSA_FLUX_ENGQUIST_OSHER)
+        return launch_step_wave<PSA_FLUX_ENGQUIST_OSHER, 0>(a, stream);
+      return launch_step_wave<PSA_FLUX_ADVECTION_UPWIND, 1>(a, stream);
+    }
+  }
   if (a.rec3) return launch_step_rec<T, 1>(d, a, cfg, stream);
   if (a.muscl) return launch_step_rec<T, 2>(d, a, cfg, stream);
   if (a.muscls) return launch_step_rec<T, 3>(d, a, cfg, stream);

@@ -657,6 +657,32 @@ def test_march_bit_for_bit(torch_mod, kind: str, dtype_name: str, n: int) -> Non
         assert torch.equal(a[k], b[k])
 
 
+@pytest.mark.parametrize("kind", ["rusanov", "godunov", "eo", "advection"])
+@pytest.mark.parametrize("n", [(1 << 21) - 1, 1 << 21, 1441 * 1456 - 6, 1441 * 1456 - 5,
+                               1441 * 1456 + 358])
+def test_step_on_wave_tiles_bit_for_bit(torch_mod, kind: str, n: int) -> None:
+    """Large FP64 states on wave tiles (workgroups of 1456 cells: last ones that
+    are full, of one cell and of one wave and a cell) compute exactly what the
+    LDS tiles compute, over the call sequence of _schedule_run."""
+    torch = torch_mod
+    from pyshocks_amd import _lib, make_uniform_cell_grid
+    from pyshocks_amd.timestepping import fused_plan
+
+    grid = make_uniform_cell_grid(0.0, 1.0, n, nghosts=3)
+    vel = torch.ones(grid.n, dtype=torch.float64, device="cuda") \
+        if kind == "advection" else None
+    plan = fused_plan(_stepper(torch, kind, grid, vel=vel,
+                               theta=0.5 if kind == "advection" else 1.0))
+    x = (torch.arange(n, dtype=torch.float64, device="cuda") + 0.5) / n
+    u = 0.4 + torch.sin(2 * torch.pi * x) + 0.5 * (x > 0.6)
+    u0 = torch.cat([u[-3:], u, u[:3]])
+    a = _schedule_run(torch, plan, u0, _lib.PSA_SCHEDULE_STEP)
+    b = _schedule_run(torch, plan, u0, _lib.PSA_SCHEDULE_DEFAULT)
+    assert a[2] == b[2]
+    for k in (0, 1):
+        assert torch.equal(a[k], b[k])
+
+
 @pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 6, 511, 512, 513, 1024, 4099])
 @pytest.mark.parametrize("offset", [0, 1])
 def test_reconstruct_pair_edges(torch_mod, n: int, offset: int) -> None:
