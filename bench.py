@@ -9,7 +9,7 @@ CFL time step); the workload's 100 steps are
 the default ``--steps``. ``value`` is cell-updates/s = N * steps / wall
 time with the state resident in HBM.
 
-A step runs as one whole-step kernel (the three stages of each tile in LDS,
+A step runs as one whole-step kernel (the three stages of each tile on chip,
 2 words of HBM traffic per cell-update) where it applies. Also reported:
 the roofline of the dominant kernel (the whole-step kernel is VALU-bound:
 executed flops per cell-update from the committed rocprofv3 counters over
