@@ -105,15 +105,14 @@ __global__ void k_weno_reconstruct(const T *__restrict__ f, int64_t m, T eps,
   }
 }
 
-// The same for WENO-JS5 in FP64 by the fused kernels' form (reconstruct_cells:
-// one reciprocal for both sides instead of twelve divisions, the reference form
-// where its denominator leaves the normal range), two cells per thread with
-// 16-byte accesses where the arrays are aligned. Bound by memory, 3 words per
-// cell; 4000043 cells: 17.5 us, one cell per thread in the reference form 41.5.
-// (FP32 keeps the reference form: its divisions are exact to the last bit, the
-// fused form's hardware reciprocals are not.)
+// The same for WENO-JS5 in FP64 with one reciprocal for both sides instead of
+// twelve divisions (weno_convex_pair; the reference form where its denominator
+// leaves its range), two cells per thread with 16-byte accesses where the arrays
+// are aligned. Bound by memory, 3 words per cell; 4000043 cells: 16.8 us, one cell
+// per thread in the reference form 41.5. (FP32 keeps the reference form: its
+// divisions are exact to the last bit, hardware reciprocals are not.)
 __global__ __launch_bounds__(256) void k_weno_reconstruct_pair(
-    StageArgs<double> p, const double *__restrict__ f, int64_t m, int aligned,
+    const double *__restrict__ f, int64_t m, double eps, int aligned,
     double *__restrict__ ul, double *__restrict__ ur) {
   const int64_t i = 2 * (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x);
   if (i >= m) return;
@@ -129,8 +128,13 @@ __global__ __launch_bounds__(256) void k_weno_reconstruct_pair(
 #pragma unroll
     for (int k = 0; k < 6; ++k) w[k] = load_raw(f, i - 2 + k, m);
   }
-  const MlpSource none{nullptr, nullptr};
-  reconstruct_cells<double, 2, false>(p, w, l, r, none, nullptr);
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    if (!weno_convex_pair(w + k, eps, l[k], r[k])) {
+      r[k] = weno_side_ref(w[k], w[k + 1], w[k + 2], w[k + 3], w[k + 4], eps);
+      l[k] = weno_side_ref(w[k + 4], w[k + 3], w[k + 2], w[k + 1], w[k], eps);
+    }
+  }
   if (aligned && i + 2 <= m) {
     store16(ul + i, double2{l[0], l[1]});
     store16(ur + i, double2{r[0], r[1]});
@@ -1453,13 +1457,11 @@ int psa_reconstruct(int dtype, int rec, const void *f, void *ul, void *ur,
   using R2 = std::integral_constant<int, PSA_REC_ESWENO32>;
   if (dtype == PSA_FLOAT64) {
     if (rec == PSA_REC_WENOJS53) {
-      StageArgs<double> a{};
-      a.eps = eps;
       const int aligned = aligned16(static_cast<const double *>(f)) &&
                           aligned16(static_cast<double *>(ul)) &&
                           aligned16(static_cast<double *>(ur));
       hipLaunchKernelGGL(k_weno_reconstruct_pair, dim3(blocks_for(m, 2 * 256)), dim3(256),
-                         0, s, a, static_cast<const double *>(f), m, aligned,
+                         0, s, static_cast<const double *>(f), m, eps, aligned,
                          static_cast<double *>(ul), static_cast<double *>(ur));
     }
     if (rec == PSA_REC_WENOJS32) launch(0.0, R1{});

@@ -166,6 +166,49 @@ __device__ __forceinline__ void weno_pair_divide(const WenoPairSums &s, double &
   ul = (s.nl * s.sr) * inv;
 }
 
+// Both sides of a cell v (FP64) as the cell's value plus a convex sum of the
+// candidates' distances from it,
+//   ur = v2 + (wr0 (5 D1 - 2 D0) + wr1 (D1 + 2 D2) + wr2 (4 D2 - D3)) / 6,
+//   ul = v2 - (wl0 (4 D1 - D0) + wl1 (2 D1 + D2) + wl2 (5 D2 - 2 D3)) / 6
+// (weno_uhat_diff, D the first differences, each side's weights indexed by
+// their indicator), with the product weights of weno_pair_sums normalised by
+// the one reciprocal of sr sl. A candidate across a jump J enters with its
+// weight of order J^-4 only, so the error stays a rounding of the smooth side,
+// as in the reference form; a sum that starts from a fixed candidate
+// (weno_diff_divide) rounds at the size of J where that candidate crosses it.
+// False (nothing written) where sr sl and its reciprocal are not far inside the
+// normal range.
+__device__ __forceinline__ bool weno_convex_pair(const double v[5], double eps, double &ul,
+                                                 double &ur) {
+  const double D0 = v[1] - v[0], D1 = v[2] - v[1], D2 = v[3] - v[2], D3 = v[4] - v[3];
+  const double s0 = D1 - D0, s1 = D2 - D1, s2 = D3 - D2;
+  const double t0 = fma(2.0, D1, s0), t1 = D2 + D1, t2 = fma(-2.0, D2, s2);
+  // 4 (eps + beta_k)
+  const double a0x4 = Weno5Coeffs<double>::a0x4, eps4 = 4.0 * eps;
+  const double e0 = fma(t0, t0, fma(a0x4, s0 * s0, eps4));
+  const double e1 = fma(t1, t1, fma(a0x4, s1 * s1, eps4));
+  const double e2 = fma(t2, t2, fma(a0x4, s2 * s2, eps4));
+  const double q0 = e0 * e0, q1 = e1 * e1, q2 = e2 * e2;
+  const double p01 = q0 * q1, p12 = q1 * q2, w1 = 6.0 * (q0 * q2);
+  const double wr2 = 3.0 * p01, wl2 = 3.0 * p12;
+  const double sr = (p12 + w1) + wr2, sl = (p01 + w1) + wl2;
+  const double den = sr * sl;
+  if (!(den > 1.0e-290 && den < 1.0e290)) return false;
+  double inv = __builtin_amdgcn_rcp(den);
+  double e = fma(-den, inv, 1.0);
+  inv = fma(inv, e, inv);
+  e = fma(-den, inv, 1.0);
+  inv = fma(inv, e, inv);
+  const double ir = sl * inv, il = sr * inv;  // 1 / sr, 1 / sl
+  const double dr = fma(wr2 * ir, fma(4.0, D2, -D3),
+                        fma(w1 * ir, fma(2.0, D2, D1), (p12 * ir) * fma(5.0, D1, -2.0 * D0)));
+  const double dl = fma(p01 * il, fma(5.0, D2, -2.0 * D3),
+                        fma(w1 * il, fma(2.0, D1, D2), (wl2 * il) * fma(4.0, D1, -D0)));
+  ur = fma(dr, 1.0 / 6.0, v[2]);
+  ul = fma(dl, -1.0 / 6.0, v[2]);
+  return true;
+}
+
 // Third-difference form of both sides (FP64, the fused kernels). With the
 // first differences D(c) = u(c) - u(c-1), the second d2(c) = D(c+1) - D(c)
 // and the third T0 = d2(c) - d2(c-1), T1 = d2(c+1) - d2(c), the candidates of

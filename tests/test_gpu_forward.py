@@ -722,6 +722,39 @@ def test_reconstruct_pair_edges(torch_mod, n: int, offset: int) -> None:
     assert (out == 9.0).all()
 
 
+@pytest.mark.parametrize("jump", [0.0, 1.0, 10.0, 1.0e3, 1.0e6])
+def test_reconstruct_beside_a_jump(torch_mod, jump: float) -> None:
+    """The FP64 reconstruction's error is a rounding of the cell's own value also
+    beside a much larger one: the candidate across the jump has a weight of
+    order jump^-4, and none of its size may enter. Against 80-bit arithmetic with
+    the coefficients in 80 bits; the last addition rounds by 2^-53 |value| and
+    the distance from the cell's value, some 20 roundings of at most a fifth of it
+    here: 5 * 2^-53 |value| at most."""
+    torch = torch_mod
+    import dataclasses
+
+    from oracle import weno_np as W
+    from pyshocks_amd import _lib
+
+    n = 48
+    ld = np.longdouble
+    f = 1.0 + 0.3 * np.sin(2 * np.pi * np.arange(n) / n + 0.3)
+    f[15:27] += jump
+    x = torch.tensor(f, device="cuda")
+    out = torch.empty((2, n), dtype=torch.float64, device="cuda")
+    _lib.call("psa_reconstruct", _lib.PSA_FLOAT64, _lib.PSA_REC_WENOJS53, _lib.ptr(x),
+              _lib.ptr(out[0]), _lib.ptr(out[1]), n, 1e-6, _lib.stream_of(x))
+    s = W.WENOJS53
+    exact = dataclasses.replace(s, a=np.round(12 * s.a).astype(ld) / 12,
+                                c=np.round(6 * s.c).astype(ld) / 6,
+                                d=np.round(10 * s.d).astype(ld) / 10)
+    ref = W.reconstruct_wenojs(f.astype(ld), ld(1e-6), exact)
+    for got, want in zip(out.cpu().numpy(), ref):
+        # (cells whose stencil lies in the array)
+        err = np.abs((got[2:-2] - want[2:-2]) / want[2:-2])
+        assert err.max() <= 5 * 2.0**-53
+
+
 @pytest.mark.parametrize("dtype_name", ["float64", "float32"])
 @pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 4095, 4097, 1 << 21, (1 << 21) + 5])
 def test_max_abs_edges(torch_mod, dtype_name: str, n: int) -> None:
