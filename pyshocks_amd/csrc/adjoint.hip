@@ -61,8 +61,8 @@ __device__ __forceinline__ double rcp_refined(double x) {
 // kernels' difference form: D_k the first differences of the stencil, s_k the
 // second ones, t = (2 D1 + s0, D1 + D2, s2 - 2 D2), e_k = 4 (eps + beta_k) =
 // 4 eps + 13/3 s_k^2 + t_k^2, T0 = s1 - s0, T1 = s2 - s1;
-//   ur = u + (D1 + 2 D2) / 6 - mR,  mR = wR0 T0 / 3 + wR2 T1 / 6,
-//   ul = u - (2 D1 + D2) / 6 + mL,  mL = wL2 T1 / 3 + wL0 T0 / 6,
+//   hR_0, hR_1, hR_2 = u + (2 t0 - D1, t1 + D2, D2 - t2) / 6,
+//   hL_0, hL_1, hL_2 = u - (t0 + D1, t1 + D1, -2 t2 - D2) / 6,
 // the weights indexed by their indicator: wR_k ~ (1, 6, 3) / e_k^2, wL_k ~
 // (3, 6, 1) / e_k^2, normalised. With
 //   dur/de_k = -2 zR_k,  zR_k = wR_k (hR_k - ur) / e_k   (left alike)
@@ -71,7 +71,7 @@ __device__ __forceinline__ double rcp_refined(double x) {
 template <typename T>
 struct CellStates {
   T s[3], t[3];
-  T qR[3], qL[3];  // w_k (h_k - value) of the right and left state
+  T qR[3], qL[3];  // 6 w_k (h_k - value) of the right and left state
   T ie[3];         // 1 / e_k
   T wR0, wR2, wL0, wL2;
 };
@@ -141,13 +141,14 @@ __device__ __forceinline__ void weno_cell_indicators(const T v[5], T eps4, T &D1
     e[k] = fma(c.t[k], c.t[k], fma(C::a0x4, c.s[k] * c.s[k], eps4));
 }
 
-// Both states from the middle candidates and the weights c.wR0 .. c.wL2.
+// Both states from the middle candidates and the weights c.wR0 .. c.wL2 (the
+// learned kernels' form, mlp_combine_ideal).
 template <typename T>
 __device__ __forceinline__ void weno_cell_values(T u, T D1, T D2, const CellStates<T> &c,
-                                                 T &mR, T &mL, T &ul, T &ur) {
+                                                 T &ul, T &ur) {
   const T a = (c.s[1] - c.s[0]) * T(1.0 / 6.0), b = (c.s[2] - c.s[1]) * T(1.0 / 6.0);
-  mR = fma(c.wR0, a + a, c.wR2 * b);
-  mL = fma(c.wL2, b + b, c.wL0 * a);
+  const T mR = fma(c.wR0, a + a, c.wR2 * b);
+  const T mL = fma(c.wL2, b + b, c.wL0 * a);
   ur = fma(c.t[1] + D2, T(1.0 / 6.0), u) - mR;
   ul = fma(c.t[1] + D1, T(-1.0 / 6.0), u) + mL;
 }
@@ -163,16 +164,25 @@ __device__ __forceinline__ void weno_cell_states(const T v[5], T eps4, CellState
   c.wR2 = wR[2];
   c.wL0 = wL[0];
   c.wL2 = wL[2];
-  T mR, mL;
-  weno_cell_values(v[2], D1, D2, c, mR, mL, ul, ur);
-  // hR_k - ur = (mR - T0/3, mR, mR - T1/6), hL_k - ul = (T0/6 - mL, -mL, T1/3 - mL)
-  const T a = (c.s[1] - c.s[0]) * T(1.0 / 6.0), b = (c.s[2] - c.s[1]) * T(1.0 / 6.0);
-  c.qR[0] = wR[0] * (mR - (a + a));
-  c.qR[1] = wR[1] * mR;
-  c.qR[2] = wR[2] * (mR - b);
-  c.qL[0] = wL[0] * (a - mL);
-  c.qL[1] = -(wL[1] * mL);
-  c.qL[2] = wL[2] * ((b + b) - mL);
+  // the states: the cell's value plus a convex sum of the candidates' distances
+  // from it, so that a candidate across a jump enters with its weight only
+  const T dR = fma(wR[2], D2 - c.t[2], fma(wR[1], c.t[1] + D2, wR[0] * fma(T(2), c.t[0], -D1)));
+  const T dL = fma(wL[2], fma(T(-2), c.t[2], -D2), fma(wL[1], c.t[1] + D1, wL[0] * (c.t[0] + D1)));
+  ur = fma(dR, T(1.0 / 6.0), v[2]);
+  ul = fma(dL, T(-1.0 / 6.0), v[2]);
+  // 6 (h_k - value) as sums of weighted differences of the candidates, 6 (hR_0 -
+  // hR_1) = -2 T0, 6 (hR_2 - hR_1) = -T1, 6 (hL_0 - hL_1) = T0, 6 (hL_2 - hL_1) =
+  // 2 T1: every term across a jump carries the weight that makes it small (the
+  // difference of a candidate and the state would leave a rounding of the jump,
+  // and 1 / e_k magnifies it); the middle one from their sum, which is zero
+  const T T0 = c.s[1] - c.s[0], T1 = c.s[2] - c.s[1];
+  const T r = fma(T(-2), T0, T1), l = fma(T(-2), T1, T0);
+  c.qR[0] = wR[0] * fma(wR[2], r, -(wR[1] * (T0 + T0)));
+  c.qR[2] = -(wR[2] * fma(wR[0], r, wR[1] * T1));
+  c.qR[1] = -(c.qR[0] + c.qR[2]);
+  c.qL[0] = wL[0] * fma(wL[2], l, wL[1] * T0);
+  c.qL[2] = wL[2] * fma(wL[1], T1 + T1, -(wL[0] * l));
+  c.qL[1] = -(c.qL[0] + c.qL[2]);
 }
 
 // cR dur/dv + cL dul/dv of a cell: through the weights (z_k = (cR qR_k +
@@ -186,7 +196,7 @@ __device__ __forceinline__ void weno_cell_scatter(const CellStates<T> &c, T cR, 
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const T z = fixed ? T(0)
-                      : T(-4) * (fma(cR, c.qR[k], cL * c.qL[k]) * c.ie[k]);
+                      : T(-2.0 / 3.0) * (fma(cR, c.qR[k], cL * c.qL[k]) * c.ie[k]);
     at[k] = z * c.t[k];
     as[k] = T(13.0 / 3.0) * (z * c.s[k]);
   }
@@ -550,8 +560,7 @@ __device__ __forceinline__ T vjp_block(const VjpArgs<T> &p, const T *s_u,
     c.wR2 = c.wL0 = T(0.3);
     static_assert(5 * B >= 14 * kLearnedRound, "the scatter's scratch holds a round");
     learned_cells_grad(sc.net, regime == 2, s_u, v, &sc.P[0][0], c, gR, gL);
-    T mR, mL;
-    weno_cell_values(v[2], D1, D2, c, mR, mL, ul, ur);
+    weno_cell_values(v[2], D1, D2, c, ul, ur);
     if (regime == 0) weno_cell_states(v, p.eps4, c, ul, ur);
   } else {
     weno_cell_states(v, p.eps4, c, ul, ur);

@@ -88,6 +88,50 @@ def test_operator_vjp_vs_complex_step(torch_mod, kind: str) -> None:
     np.testing.assert_array_equal(got[-3:], 0.0)
 
 
+@pytest.mark.parametrize("velocity", [1.0, -1.0])
+@pytest.mark.parametrize("jump", [0.1, 10.0, 100.0])
+def test_operator_vjp_beside_a_jump(torch_mod, monkeypatch, velocity: float,
+                                    jump: float) -> None:
+    """The gradient of one side's states keeps its digits beside a much larger
+    value: the candidate across the jump has a weight of order jump^-4, and the
+    small 1 / (eps + beta) of the smooth side must not meet a rounding of the
+    jump. Against the complex step in 80 bits with the coefficients in 80 bits
+    (whose own cancellation, the reference form's, is below 1e-15 for these jumps);
+    some 40 roundings lie between the stencil and an entry: 40 * 2^-53 of the
+    largest."""
+    torch = torch_mod
+    import dataclasses
+
+    from oracle import adjoint_cs as A
+    from oracle import weno_np as W
+    from pyshocks_amd.adjoint import operator_vjp
+
+    ld = np.longdouble
+    s = W.WENOJS53
+    exact = dataclasses.replace(s, a=np.round(12 * s.a).astype(ld) / 12,
+                                c=np.round(6 * s.c).astype(ld) / 6,
+                                d=np.round(10 * s.d).astype(ld) / 10)
+    monkeypatch.setattr(A, "_reconstruct_cs",
+                        lambda f, eps: W.reconstruct_wenojs(f, ld(eps), exact))
+    n, g = 40, 3
+    grid = W.make_uniform_cell_grid(0.0, 1.0, n, nghosts=g)
+    u = 1.0 + 0.3 * np.sin(2 * np.pi * (np.arange(n + 2 * g) - 2.5) / n + 0.3)
+    u[15:27] += jump
+    u = W.apply_boundary_periodic(grid, u)
+    mu = np.random.default_rng(1).standard_normal(n + 2 * g)
+    src, _ = _source(torch, "advection", n, velocity)
+    got = _host(operator_vjp(src, _dev(torch, u), _dev(torch, mu)))
+    ref = np.empty(n, dtype=ld)
+    h = ld(1.0e-30)
+    for j in range(n):
+        z = u.astype(np.clongdouble)
+        z[g + j] += 1j * h
+        z = W.apply_boundary_periodic(grid, z)
+        out = A.apply_operator_cs("advection", grid, z, eps=1e-6, velocity=velocity)
+        ref[j] = (out[g:g + n].imag / h) @ mu[g:g + n]
+    assert np.abs(got[g:-g] - ref).max() <= 40 * 2.0**-53 * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("kind", KINDS_LF)
 @pytest.mark.parametrize("n", [40, 600])
 def test_step_vjp_vs_complex_step(torch_mod, kind: str, n: int) -> None:
