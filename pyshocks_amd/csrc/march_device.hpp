@@ -343,7 +343,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     }
   }
   if (tile == 0 && tid < 64) {
-    if (from_state) ctrl->umax_slot[tid][0] = tid == 0 ? umax : 0ull;
+    // (without a step, tiles that start later still read the slots: a mixture of
+    // old and new ones could have them take a step that the others do not)
+    if (from_state && taken) ctrl->umax_slot[tid][0] = tid == 0 ? umax : 0ull;
     if (tid == 0) {
       ctrl->t = t;
       ctrl->m = mstep;

@@ -806,6 +806,33 @@ def test_march_lax_friedrichs_bit_for_bit(torch_mod, dtype_name: str, n: int) ->
         assert torch.equal(a[k], b[k])
 
 
+@pytest.mark.parametrize("kind", ["rusanov", "lf"])
+@pytest.mark.parametrize("why", ["time", "nan"])
+def test_march_first_step_not_taken(torch_mod, kind: str, why: str) -> None:
+    """A call of many steps in one launch that takes none (the final time is
+    reached; the maximum is NaN) copies the state with its ghost cells as given,
+    and leaves the control block's maximum, partials in several slots which the
+    tiles read at different times, as it is."""
+    torch = torch_mod
+    from pyshocks_amd import _lib, make_uniform_cell_grid
+    from pyshocks_amd.timestepping import fused_plan
+
+    n = 40000
+    plan = fused_plan(_stepper(torch, kind, make_uniform_cell_grid(0.0, 1.0, n, nghosts=3)))
+    u = torch.linspace(-1.0, 2.0, n + 6, dtype=torch.float64, device="cuda")
+    if why == "nan":
+        u[n // 2] = float("nan")
+    ctrl = plan.new_control(u, 0.0, 0.0 if why == "time" else float("inf"), None)
+    before = plan.read_control(ctrl)
+    x = torch.full_like(u, 7.0)
+    plan.steps(u, x, torch.empty_like(u), torch.empty_like(u), ctrl, 8)
+    after = plan.read_control(ctrl)
+    assert after.m == 0 and after.t == 0.0 and after.active == 0
+    assert after.status == (_lib.PSA_OK if why == "time" else _lib.PSA_ERR_NONFINITE_DT)
+    assert max(s[0] for s in after.umax_slot) == max(s[0] for s in before.umax_slot)
+    assert torch.equal(x.view(torch.int64), u.view(torch.int64))
+
+
 def test_march_in_a_graph(torch_mod) -> None:
     """A captured call of many steps in one launch, replayed on a running
     control block with eager work in between, continues the eager run's
