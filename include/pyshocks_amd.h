@@ -346,7 +346,11 @@ typedef struct psa_solver_desc {
                                    whole-step kernel of psa_ssprk33_steps
                                    fills the ghost cells of every stage
                                    input itself (below)                    */
-  int pad3_;
+  int march_wait_us;            /* steps of a call in one launch of several
+                                   workgroups (PSA_SCHEDULE_DEFAULT below):
+                                   how long it waits for all of them to be
+                                   running, 0: a second, negative: it does
+                                   not try                                 */
   double es_delta;              /* PSA_FLUX_ESWENO: delta of the
                                    dissipative flux                        */
   /* PSA_BC_NEUMANN (scalar.py:466-511 with a constant g on each side): the
@@ -389,7 +393,16 @@ typedef struct psa_solver_desc {
  *   mid-size periodic state without learned weights or Rusanov nu (up to
  *   505856 cells; MUSCL 243712; Lax-Friedrichs in FP32 1030144; default tiles),
  *   one launch whose workgroups hold a tile each and exchange edges and
- *   maxima through k2, else STEP where it applies, else TILE.
+ *   maxima through k2 (where k2 holds the words, 1152 bytes a workgroup in FP64 and
+ *   640 in FP32), else STEP where it applies, else TILE.
+ *   Those workgroups wait for each other, so all have to be on the device at once.
+ *   The launch takes at most a quarter of what the device holds, which leaves room
+ *   for four such calls at a time. Where it does not get its place within
+ *   march_wait_us (more of them, other processes' kernels, a stream restricted to
+ *   few CUs), its workgroups leave with nothing done and a launch of one
+ *   workgroup takes the steps of the call: the same values, on one CU. A program
+ *   that runs many such calls at a time takes PSA_SCHEDULE_STEP, whose launches
+ *   wait for nothing.
  * All schedules compute the same values. */
 #define PSA_SCHEDULE_DEFAULT 0
 #define PSA_SCHEDULE_TILE 1
@@ -425,9 +438,9 @@ int psa_ssprk33_steps(const psa_solver_desc *desc, const void *u_in,
                       long long nsteps, void *stream);
 
 /* 1 if a psa_ssprk33_steps call of 4 or more steps on this descriptor (with a
- * valid control block) runs them all in one launch, which ends with the last
- * step that is taken, so that enqueuing more steps than a run needs costs
- * nothing; 0 if not. */
+ * valid control block) runs them all in one launch (with at most two short ones
+ * beside it), which ends with the last step that is taken, so that enqueuing more
+ * steps than a run needs costs nothing; 0 if not. */
 int psa_ssprk33_one_launch(const psa_solver_desc *desc);
 
 /* One stage (1, 2 or 3) of timestepping.py:312-320: stage 1 out = uk + dt L(uk),

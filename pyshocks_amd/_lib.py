@@ -126,7 +126,7 @@ class PsaSolverDesc(ctypes.Structure):
         ("limiter_theta", ctypes.c_double),
         ("muscl_atol", ctypes.c_double),
         ("bc", ctypes.c_int),
-        ("pad3_", ctypes.c_int),
+        ("march_wait_us", ctypes.c_int),
         ("es_delta", ctypes.c_double),
         ("bc_left", ctypes.c_double),
         ("bc_right", ctypes.c_double),

@@ -1242,7 +1242,7 @@ int run_steps(const psa_solver_desc *d, const void *u_in, void *u_out,
   if (a.ctrl != nullptr && nsteps >= kMarchLeastSteps && march_applies(d, cfg, vel)) {
     a.uk = un;
     a.out = uo;
-    st = launch_march(d, a, nsteps, b2, stream);
+    st = launch_march(d, a, nsteps, b1, b2, stream);
     if (st != PSA_ERR_NOT_IMPLEMENTED) return st;
   }
   if (a.ctrl != nullptr && step_applies(d, cfg, vel)) {
@@ -1927,8 +1927,10 @@ int psa_ssprk33_one_launch(const psa_solver_desc *desc) {
   if (ring_applies(desc, vel)) return 1;
   if (!march_applies(desc, tiles_of(desc), vel)) return 0;
   const int st = desc->dtype == PSA_FLOAT64
-                     ? launch_march(desc, make_args<double>(desc), 0, nullptr, nullptr)
-                     : launch_march(desc, make_args<float>(desc), 0, nullptr, nullptr);
+                     ? launch_march(desc, make_args<double>(desc), 0, nullptr, nullptr,
+                                    nullptr)
+                     : launch_march(desc, make_args<float>(desc), 0, nullptr, nullptr,
+                                    nullptr);
   return st == PSA_OK ? 1 : 0;
 }
 

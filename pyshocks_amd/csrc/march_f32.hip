@@ -4,8 +4,8 @@
 namespace psa {
 
 int launch_march(const psa_solver_desc *d, const StageArgs<float> &a, long long nsteps,
-                 void *scratch, hipStream_t s) {
-  return launch_march_t<float>(d, a, nsteps, scratch, s);
+                 void *k1, void *k2, hipStream_t s) {
+  return launch_march_t<float>(d, a, nsteps, k1, k2, s);
 }
 
 }  // namespace psa

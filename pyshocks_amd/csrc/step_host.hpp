@@ -126,9 +126,10 @@ int launch_ring(const psa_solver_desc *d, const StageArgs<double> &a, long long 
 int launch_ring(const psa_solver_desc *d, const StageArgs<float> &a, long long nsteps,
                 hipStream_t stream);
 
-// Steps below which its two launches are not worth it (us a step as launches and
-// as a march, N = 16384: one step 15.4, 15.7, two 10.4, 10.8, four 7.9, 6.7), and
-// the cells that a tile's margins need.
+// Steps below which its three launches are not worth it (FP64, us a step as
+// launches and as a march in calls of four: N = 1500 6.0, 4.2; 16384 6.0, 4.6;
+// 374784 8.0, 7.7; 505856 9.0, 9.3, in calls of eight 8.4, 8.1), and the cells that
+// a tile's margins need.
 constexpr long long kMarchLeastSteps = 4;
 constexpr int64_t kMarchLeastCells = 64;
 
@@ -143,14 +144,14 @@ inline bool march_applies(const psa_solver_desc *d, TileConfig cfg, int vel) {
           (d->flux == PSA_FLUX_LAX_FRIEDRICHS && d->nu == nullptr));
 }
 
-// The steps of a call as a march; scratch: an array of m cells of the state's
-// type. PSA_ERR_NOT_IMPLEMENTED (nothing launched) where the state is too large
-// for it or the device too small. With a null scratch: the same answer, and
+// The steps of a call as a march; k1, k2: scratch arrays of m cells of the
+// state's type. PSA_ERR_NOT_IMPLEMENTED (nothing launched) where the state is too
+// large for it or the device too small. With a null k2: the same answer, and
 // nothing is launched.
 int launch_march(const psa_solver_desc *d, const StageArgs<double> &a, long long nsteps,
-                 void *scratch, hipStream_t stream);
+                 void *k1, void *k2, hipStream_t stream);
 int launch_march(const psa_solver_desc *d, const StageArgs<float> &a, long long nsteps,
-                 void *scratch, hipStream_t stream);
+                 void *k1, void *k2, hipStream_t stream);
 
 // Workgroups the device holds at once for a kernel (CUs x occupancy),
 // queried once per kernel and device (the kernel is the template argument,

@@ -806,6 +806,87 @@ def test_march_lax_friedrichs_bit_for_bit(torch_mod, dtype_name: str, n: int) ->
         assert torch.equal(a[k], b[k])
 
 
+def _march_run(torch, plan, u0, sched: int):
+    """Calls of many steps on one schedule: in place, out of place on the same
+    control block, one that stops after six or more steps, and one whose first
+    step is not taken; the states and (t, dt, m, status, max|u|) after each."""
+    plan.desc.schedule = sched
+    big = float(np.finfo(plan.np_dtype).max)
+    u, k1, k2 = u0.clone(), torch.empty_like(u0), torch.empty_like(u0)
+    v, w, x = (torch.full_like(u0, 7.0) for _ in range(3))
+    ctrl = plan.new_control(u, 0.0, big, None)
+    fields = []
+
+    def call(a, b, c, n):
+        plan.steps(a, b, k1, k2, c, n)
+        r = plan.read_control(c)
+        fields.append((r.t, r.dt, r.m, r.status, r.active, max(s[0] for s in r.umax_slot)))
+        return r
+
+    call(u, u, ctrl, 9)
+    c = call(u, v, ctrl, 8)
+    assert c.m == 17 and c.status == 0 and c.active == 1
+    ctrl2 = plan.new_control(v, 0.0, 6.5 * c.dt, None)
+    c2 = call(v, w, ctrl2, 16)
+    assert 6 <= c2.m < 16 and c2.status == 0 and c2.active == 0
+    c3 = call(w, x, ctrl2, 8)
+    assert c3.m == c2.m and c3.active == 0 and torch.equal(x, w)
+    return (u, v, w), fields
+
+
+def _march_scheme(torch, kind: str, n: int, dtype):
+    """The fused plan of a flux ("rusanov", .., "lf"), or of a reconstruction under
+    Rusanov, or "esweno-flux"; a state with its ghost cells."""
+    from oracle import exact as E
+    from pyshocks_amd import bind, burgers, make_uniform_cell_grid
+    from pyshocks_amd.limiters import make_limiter_from_name
+    from pyshocks_amd.reconstruction import ESWENO32, make_reconstruction_from_name
+    from pyshocks_amd.scalar import PeriodicBoundary
+    from pyshocks_amd.timestepping import fused_plan, make_ssprk33
+
+    grid = make_uniform_cell_grid(0.0, 1.0, n, nghosts=3, dtype=dtype)
+    bc = PeriodicBoundary()
+    if kind in ("wenojs32", "esweno32"):
+        sch = burgers.Rusanov(rec=make_reconstruction_from_name(kind, eps=1e-6))
+    elif kind in ("muscl", "muscls"):
+        lm = make_limiter_from_name("minmod", theta=1.0, variant=1)
+        sch = burgers.Rusanov(rec=make_reconstruction_from_name(kind, lm=lm))
+    elif kind == "esweno-flux":
+        sch = bind(burgers.ESWENO32(rec=ESWENO32()), grid, bc)
+    else:
+        sch = None
+    if sch is None:
+        vel = torch.ones(grid.n, dtype=dtype, device="cuda") if kind == "advection" else None
+        st = _stepper(torch, kind, grid, vel=vel, theta=0.5 if kind == "advection" else 1.0)
+    else:
+        st = make_ssprk33(sch, grid, bc, theta=1.0)
+    u0 = torch.tensor(E.exact_cell_averages(E.large_initial_condition(seed=6), n),
+                      device="cuda").to(dtype)
+    return fused_plan(st), u0
+
+
+@pytest.mark.parametrize("kind", ["rusanov", "advection", "lf", "wenojs32", "muscl", "muscls",
+                                  "esweno-flux"])
+@pytest.mark.parametrize("dtype_name", ["float64", "float32"])
+@pytest.mark.parametrize("n", [1200, 20001])
+@pytest.mark.parametrize("wait_us", [-1, 1])
+def test_march_given_up(torch_mod, kind: str, dtype_name: str, n: int, wait_us: int) -> None:
+    """A call in one launch whose workgroups do not all start in time leaves the
+    steps to one workgroup, which computes the same bits: always (a negative wait)
+    and, with a wait of a microsecond, in whichever calls it happens."""
+    torch = torch_mod
+    from pyshocks_amd import _lib
+
+    plan, u0 = _march_scheme(torch, kind, n, getattr(torch, dtype_name))
+    assert plan.runs_in_one_launch()
+    a = _march_run(torch, plan, u0, _lib.PSA_SCHEDULE_DEFAULT)
+    plan.desc.march_wait_us = wait_us
+    b = _march_run(torch, plan, u0, _lib.PSA_SCHEDULE_DEFAULT)
+    assert a[1] == b[1]
+    for p, q in zip(a[0], b[0]):
+        assert torch.equal(p, q)
+
+
 @pytest.mark.parametrize("kind", ["rusanov", "lf"])
 @pytest.mark.parametrize("why", ["time", "nan"])
 def test_march_first_step_not_taken(torch_mod, kind: str, why: str) -> None:
