@@ -544,17 +544,25 @@ def _step_generic(stepper: Stepper, u0: torch.Tensor, *, maxit: int | None,
 ONE_LAUNCH_STEPS = 16384
 
 
+class _Default(int):
+    """The default of an argument, told apart from the same number given."""
+
+
+DEFAULT_CHUNK = _Default(64)
+
+
 def evolve(stepper: Stepper, u0: torch.Tensor, *, maxit: int | None = None,
            tstart: float = 0.0, tfinal: float | None = None,
-           chunk: int = 64, tiles: tuple[int, int] | None = None) -> StepCompleted:
+           chunk: int = DEFAULT_CHUNK,
+           tiles: tuple[int, int] | None = None) -> StepCompleted:
     """Run :func:`step` to completion without per-step host synchronisation
     and return the final :class:`StepCompleted`.
 
     Steps are enqueued ``chunk`` at a time (one chunk of exactly ``maxit``
-    steps when only ``maxit`` bounds the run; at least ``ONE_LAUNCH_STEPS``
-    where they run in one launch that ends with the run) and the device-side
-    control block is read back once per chunk. ``u0`` is not modified. ``tiles``
-    as in :func:`fused_plan`.
+    steps when only ``maxit`` bounds the run; by default 64, or
+    ``ONE_LAUNCH_STEPS`` where they run in one launch that ends with the run) and
+    the device-side control block is read back once per chunk. ``u0`` is not
+    modified. ``tiles`` as in :func:`fused_plan`.
     """
     plan = fused_plan(stepper, tiles=tiles)
     if plan is None:
@@ -578,8 +586,8 @@ def evolve(stepper: Stepper, u0: torch.Tensor, *, maxit: int | None = None,
     # steps past the end of the run cost nothing where one launch runs them all
     # (N = 256 to t = 0.5, 368 steps: about 370 us in
     # chunks of 64, 274 at once)
-    if plan.runs_in_one_launch():
-        chunk = max(chunk, ONE_LAUNCH_STEPS)
+    if chunk is DEFAULT_CHUNK and plan.runs_in_one_launch():
+        chunk = ONE_LAUNCH_STEPS
     c = None
     while True:
         m = 0 if c is None else int(c.m)

@@ -432,3 +432,51 @@ def test_batched_team_size_argument_checked_before_any_allocation() -> None:
     for bad in (-1, 2.5, True, "cells"):
         with pytest.raises(ValueError, match="team_cells"):
             BatchedSolver([64, 128], team_cells=bad)
+
+
+def test_evolve_chunk(monkeypatch) -> None:
+    """evolve enqueues as many steps at a time as its caller asks for, also where
+    one launch would run them all; only by default does it choose itself."""
+    import inspect
+    import types
+
+    import torch
+
+    from pyshocks_amd import _lib, timestepping
+
+    class Plan:
+        np_dtype = np.float64
+
+        def __init__(self, one_launch: bool) -> None:
+            self.one_launch, self.calls, self.m = one_launch, [], 0
+
+        def new_control(self, *args):
+            return None
+
+        def runs_in_one_launch(self) -> bool:
+            return self.one_launch
+
+        def steps(self, u_in, u_out, k1, k2, ctrl, n: int) -> None:
+            self.calls.append(n)
+            self.m = min(self.m + n, 100)
+
+        def read_progress(self, ctrl):
+            return types.SimpleNamespace(t=0.0, dt=1.0, m=self.m, status=_lib.PSA_OK,
+                                         active=int(self.m < 100))
+
+    monkeypatch.setattr(_lib, "require_device", lambda *a: None)
+
+    def calls(one_launch: bool, **kwargs) -> list[int]:
+        plan = Plan(one_launch)
+        monkeypatch.setattr(timestepping, "fused_plan", lambda *a, **k: plan)
+        end = timestepping.evolve(None, torch.zeros(10, dtype=torch.float64), tfinal=1.0,
+                                  **kwargs)
+        assert end.iteration == 100
+        return plan.calls
+
+    assert inspect.signature(timestepping.evolve).parameters["chunk"].default == 64
+    assert calls(False) == [64, 64]
+    assert calls(True) == [timestepping.ONE_LAUNCH_STEPS]
+    for one_launch in (False, True):
+        assert calls(one_launch, chunk=64) == [64, 64]
+        assert calls(one_launch, chunk=40) == [40, 40, 40]
