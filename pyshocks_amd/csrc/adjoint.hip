@@ -391,7 +391,7 @@ __device__ __forceinline__ void learned_network(VjpNet<T, true> &net, const T *s
 #pragma unroll
   for (int k = 0; k < 5; ++k) a1 = fma(w1[k], left ? x[4 - k] : x[k], a1);
   hb[unit] = a1 > T(0) ? a1 : T(0);
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_handover();
   T acc[4] = {net.b2[unit], T(0), T(0), T(0)};
 #pragma unroll 8
   for (int j = 0; j < MLP_HID; ++j) acc[j & 3] = fma(net.w2[unit][j], hb[j], acc[j & 3]);
@@ -413,9 +413,9 @@ __device__ __forceinline__ void learned_network(VjpNet<T, true> &net, const T *s
   const T sw = c0 * p0 + c2 * p2;
   const T hb2 =
       fma(w3[0], p0 * (c0 - sw), fma(w3[1], p1 * (T(0) - sw), w3[2] * (p2 * (c2 - sw))));
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_handover();
   hb[unit] = a2 > T(0) ? hb2 : T(0);
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_handover();
   T bcc[4] = {T(0), T(0), T(0), T(0)};
 #pragma unroll 8
   for (int i = 0; i < MLP_HID; ++i) bcc[i & 3] = fma(net.w2[i][unit], hb[i], bcc[i & 3]);
@@ -423,7 +423,7 @@ __device__ __forceinline__ void learned_network(VjpNet<T, true> &net, const T *s
   hb1 = a1 > T(0) ? hb1 : T(0);
 #pragma unroll
   for (int k = 0; k < 5; ++k) xb[k] = half_sum(w1[k] * hb1);
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_handover();
 }
 
 // What the network adds to the states of the learned cells of a workgroup:

@@ -245,9 +245,7 @@ __global__ __launch_bounds__(GRAD_BLOCK) void k_mlp_grad(
 
     // ---- parameter gradients: sums over the wave's samples (its own LDS
     // rows, so the wave's own order is enough)
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_handover();
     const int u32 = lane & 31, k2 = lane >> 5;
 #pragma unroll
     for (int t = 0; t < GRAD_SPW; t += 2) {
@@ -269,7 +267,7 @@ __global__ __launch_bounds__(GRAD_BLOCK) void k_mlp_grad(
                                                       0, 0);
       }
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_handover();  // (the next pass writes the rows again)
   }
 
   // ---- the waves' sums, then their sum in wave order

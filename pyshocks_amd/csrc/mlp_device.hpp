@@ -52,6 +52,17 @@
 
 namespace psa {
 
+// Hands LDS values from lane to lane within a wave: what the lanes stored before
+// it is there for every lane's loads after it, and loads before it are done before
+// stores after it. The barrier alone orders the instructions, not the memory; at
+// this scope the fences cost no instructions (a wave's LDS accesses are in
+// order).
+__device__ __forceinline__ void wave_lds_handover() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
