@@ -637,7 +637,9 @@ def test_march_bit_for_bit(torch_mod, kind: str, dtype_name: str, n: int) -> Non
     """The steps of a call in one launch (the default schedule of mid-size
     periodic states: full and barely more than full tiles of one to eight
     cells per lane, and the first size above them) compute exactly what the
-    whole-step kernel computes, over the call sequence of _schedule_run."""
+    whole-step kernel computes, over the call sequence of _schedule_run, of which
+    the call of 8 steps is one launch that takes the first two (many steps:
+    test_march_many_steps)."""
     torch = torch_mod
     from oracle import exact as E
     from pyshocks_amd import _lib, make_uniform_cell_grid
@@ -691,7 +693,8 @@ def test_reconstruct_pair_edges(torch_mod, n: int, offset: int) -> None:
     beside them. Six indicators, products and the reciprocal leave some 20
     roundings in a weight and the candidates are at most 10/3 max|f|, twice (the
     oracle rounds too): 2 * 20 * 10/3 * 2^-53 max|f| at most, of which the sums'
-    cancellation shows a tenth."""
+    cancellation shows a tenth. (The scale is the stencil's largest value; the error
+    beside it in test_reconstruct_beside_a_jump.)"""
     torch = torch_mod
     from oracle import weno_np as W
     from pyshocks_amd import _lib
@@ -786,7 +789,8 @@ def test_max_abs_edges(torch_mod, dtype_name: str, n: int) -> None:
 def test_march_lax_friedrichs_bit_for_bit(torch_mod, dtype_name: str, n: int) -> None:
     """Lax-Friedrichs steps of a call in one launch (one tile, several, and the
     sizes on either side of its rule) compute exactly what the stage kernels
-    compute, over the call sequence of _schedule_run."""
+    compute, over the call sequence of _schedule_run, of which the call of 8 steps
+    is one launch that takes the first two (many steps: test_march_many_steps)."""
     torch = torch_mod
     from oracle import exact as E
     from pyshocks_amd import _lib, make_uniform_cell_grid
@@ -863,6 +867,38 @@ def _march_scheme(torch, kind: str, n: int, dtype):
     u0 = torch.tensor(E.exact_cell_averages(E.large_initial_condition(seed=6), n),
                       device="cuda").to(dtype)
     return fused_plan(st), u0
+
+
+#: a size for every number of cells per lane (one, two, four, six, eight; MUSCL up
+#: to four; Lax-Friedrichs also one workgroup alone and, in FP32, sixteen)
+_MARCH_SIZES = [("float64", n) for n in (1200, 47105, 200001, 300001, 505856)]
+_MARCH_SIZES += [("float32", n) for _, n in _MARCH_SIZES]
+_MARCH_CASES = [(kind, dtype, n)
+                for kind in ("rusanov", "godunov", "eo", "advection", "lf", "wenojs32",
+                             "esweno32", "muscl", "muscls", "esweno-flux")
+                for dtype, n in _MARCH_SIZES if n <= 243712 or "muscl" not in kind]
+_MARCH_CASES += [("lf", dtype, n) for dtype in ("float64", "float32") for n in (184, 952)]
+_MARCH_CASES += [("lf", "float32", 1030144)]
+
+
+@pytest.mark.parametrize("kind,dtype_name,n", _MARCH_CASES)
+def test_march_many_steps(torch_mod, kind: str, dtype_name: str, n: int) -> None:
+    """Calls of many steps in one launch -- every set of exchange words and of edge
+    cells written again, turns of either parity, in place and out of place, a
+    second call on the control block, a stop inside a call and a call without a
+    step -- leave the bits of the whole-step kernel (Lax-Friedrichs: of the stage
+    kernels), for every flux, reconstruction and number of cells per lane."""
+    torch = torch_mod
+    from pyshocks_amd import _lib
+
+    plan, u0 = _march_scheme(torch, kind, n, getattr(torch, dtype_name))
+    assert plan.runs_in_one_launch()
+    a = _march_run(torch, plan, u0,
+                   _lib.PSA_SCHEDULE_TILE if kind == "lf" else _lib.PSA_SCHEDULE_STEP)
+    b = _march_run(torch, plan, u0, _lib.PSA_SCHEDULE_DEFAULT)
+    assert a[1] == b[1]
+    for p, q in zip(a[0], b[0]):
+        assert torch.equal(p, q)
 
 
 @pytest.mark.parametrize("kind", ["rusanov", "advection", "lf", "wenojs32", "muscl", "muscls",
