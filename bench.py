@@ -241,7 +241,8 @@ def gpu_leg(args: argparse.Namespace) -> dict:
         # one whole-step launch per step (the prologue launch of the call is
         # inside the region, ~0.01 % of it)
         kernel_ms = region_ms / args.steps
-        dominant = "k_step"
+        dominant = ("k_march" if args.steps >= 4 and plan.runs_in_one_launch() else
+                    "k_step_wave" if plan.uses_wave_tiles() else "k_step")
         algo_bytes = WHOLE_STEP_WORDS * n * itemsize
     else:
         kernel_ms = stage_ms[stage_dominant]
@@ -280,9 +281,10 @@ def _profile_entry(name: str, key: str):
 def roofline_record(args: argparse.Namespace, gpu: dict, traffic, valu) -> dict:
     """Roofline of the dominant kernel. The whole-step kernel moves 2 words
     per cell-update and is bound by the vector ALU: its executed flops (and
-    VALU instructions) per cell-update come from the rocprofv3 counters in
-    profiles/valu.json, timed live with the event-timed kernel duration; the
-    HBM figures are reported beside them. The stage kernels are HBM-bound."""
+    VALU instructions) per cell-update come from the rocprofv3 counters of the
+    kernel that runs in profiles/valu.json, timed live with the event-timed kernel
+    duration; the HBM figures are reported beside them, and alone where that kernel
+    has no counters there. The stage kernels are HBM-bound."""
     hbm_gbs = gpu["achieved_gbs"]
     hbm = {
         "achieved": hbm_gbs,
@@ -299,7 +301,8 @@ def roofline_record(args: argparse.Namespace, gpu: dict, traffic, valu) -> dict:
         "frac": gpu["stage_achieved_gbs"] / HBM_PEAK_GBS,
         "unit": "GB/s",
     }
-    if not gpu["whole_step"] or valu is None:
+    if not gpu["whole_step"] or valu is None or not valu["kernel"].startswith(
+            gpu["kernel"] + "<"):
         return {"bound": "hbm", **{k: hbm[k] for k in ("achieved", "peak", "unit", "frac",
                                                         "traffic")},
                 "kernel": gpu["kernel"], "kernel_ms": gpu["kernel_ms"],
@@ -316,7 +319,7 @@ def roofline_record(args: argparse.Namespace, gpu: dict, traffic, valu) -> dict:
         "unit": "TFLOP/s",
         "frac": tflops / peak,
         "traffic": traffic,
-        "kernel": gpu["kernel"],
+        "kernel": valu["kernel"],
         "kernel_ms": gpu["kernel_ms"],
         "flops_per_cell_update": valu["flops_per_cell_update"],
         "valu_instr_per_cell_update": valu["valu_instr_per_cell_update"],
@@ -1050,13 +1053,18 @@ def main(argv: list[str] | None = None) -> int:
     learned = None if args.no_learned else learned_leg(args)
     cpu = cpu_leg(args, gpu)
 
-    kname = "step" if gpu["whole_step"] else f"stage{gpu['stage_dominant']}"
+    kname = (gpu["kernel"].removeprefix("k_") if gpu["whole_step"]
+             else f"stage{gpu['stage_dominant']}")
     recs = "" if args.rec == "wenojs53" else f"_{args.rec}"
     if args.rec in ("muscl", "muscls"):
         recs = f"_{args.rec}_{args.limiter}"
+    if args.learned:
+        recs += "_learned"
     key = f"{args.scheme}{recs}_{args.dtype}_{args.n}_{kname}"
-    traffic = _profile_entry("traffic.json", key)
-    valu = _profile_entry("valu.json", key)
+    # (the counters are of the default tiles)
+    tuned = args.block == 0 and args.cells_per_thread == 0
+    traffic = _profile_entry("traffic.json", key) if tuned else None
+    valu = _profile_entry("valu.json", key) if tuned else None
     roofline = roofline_record(args, gpu, traffic, valu)
 
     dtype_name = "f64" if args.dtype == "f64" else "f32"
@@ -1082,7 +1090,7 @@ def main(argv: list[str] | None = None) -> int:
             "reconstruction": (f"{args.rec}-{args.limiter}" if args.rec in ("muscl", "muscls")
                                else args.rec),
             "step": ("one SSP-RK3 time step (one whole-step kernel: the three stages of "
-                     "each tile in LDS, device CFL dt)" if gpu["whole_step"] else
+                     "each tile on chip, device CFL dt)" if gpu["whole_step"] else
                      "one SSP-RK3 time step (3 fused stage kernels, device CFL dt)"),
         },
         "roofline": roofline,

@@ -378,17 +378,17 @@ typedef struct psa_solver_desc {
  * STEP: one kernel per step (a one-wave kernel before and after the call's
  *   steps); every workgroup decides the step from the control block, loads
  *   its tile of u^n with a 12-cell margin on each side, runs the three
- *   stages in LDS (recomputing the margin cells of the first two) and writes
- *   u^(n+1) (2 words per cell and step; any reconstruction, WENO-JS or
+ *   stages in LDS (recomputing the margin cells of the first two; under DEFAULT
+ *   large FP64 states in the registers of a wave per tile) and writes u^(n+1) (2 words per cell and step; any reconstruction, WENO-JS or
  *   learned weights, no velocity array, no Rusanov nu, not Lax-Friedrichs
  *   (its stages need the global max|u| of the previous stage), a control
  *   block, tiles 256 x 4 or 256 x 2). Steps ping-pong between u_out and the
  *   stage buffers.
  * RING: one launch for all the steps of the call; one workgroup holds a
- *   periodic state of n <= PSA_RING_MAX_CELLS cells in its waves' registers
- *   and takes the steps with the arithmetic and the decisions of
- *   STEP, with no HBM traffic between steps (what STEP takes, periodic, no
- *   learned weights; the stage buffers are not used).
+ *   periodic state of n <= PSA_RING_MAX_CELLS cells (in its waves' registers
+ *   within a step, in LDS from one to the next) and takes the steps with the
+ *   arithmetic and the decisions of STEP, with no HBM traffic between steps (what
+ *   STEP takes, periodic, no learned weights; the stage buffers are not used).
  * DEFAULT is RING where it applies, else, for calls of at least 4 steps on a
  *   mid-size periodic state without learned weights or Rusanov nu (up to
  *   505856 cells; MUSCL 243712; Lax-Friedrichs in FP32 1030144; default tiles),

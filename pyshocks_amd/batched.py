@@ -147,8 +147,8 @@ class BatchedSolver:
         # FP64 time keeps FP32 instances on schedule over ~10^5 steps; False
         # accumulates t in the state dtype as the reference's step loop does
         self.desc.time_f64 = 1 if time_f64 else 0
-        # one sweep per step with the three stages of a tile in LDS, or one
-        # sweep per stage (the same values)
+        # one sweep per step with the three stages of a tile in a wave's
+        # registers, or one sweep per stage (the same values)
         self.desc.schedule = _lib.PSA_SCHEDULE_STEP if schedule == "step" \
             else _lib.PSA_SCHEDULE_TILE
         self.rec = rec

@@ -5,10 +5,10 @@
 // longest instances first). A slot is one member of an instance's team: an
 // instance of team size 1 is run by one workgroup alone, a large instance by
 // a team of workgroups that split its cells and meet after every step (stage
-// sweeps: at a global barrier after every stage). Every member runs the instance's whole time loop: the
-// CFL time step of timestepping.py:89-152 with predict_timestep of
-// burgers/schemes.py:42-49,121-127 (Rusanov with alpha = 1 or Godunov), and
-// the three SSP-RK3 stages of timestepping.py:312-320, each a sweep over its
+// sweeps: at a global barrier after every stage). Every member runs the
+// instance's whole time loop: the CFL time step of timestepping.py:89-152 with
+// predict_timestep of burgers/schemes.py:42-49,121-127 (Rusanov with alpha = 1 or
+// Godunov), and the three SSP-RK3 stages of timestepping.py:312-320, each a sweep over its
 // tiles with the same tile computation as the single-instance stage kernels,
 // or the step as one sweep of wave tiles (the default schedule).
 // max|u| of each new state is reduced in the workgroup and, for a team,
@@ -235,14 +235,11 @@ __global__ __launch_bounds__(64) void k_batch_words(BatchArgs<T> a) {
 // written by themselves only; what they need of each other, nine cells on
 // either side and the maximum, goes through exchange words (in the instance's
 // k2 array), so that a step needs no write-back or invalidation of an L2, which
-// holds the states of every other workgroup of the XCD too. With fences at every
-// step and a tile per workgroup in LDS the same batches took, ms before and
-// after (default tiles): 1024 instances of 128 to 65536 cells FP32 60.0, 27.5,
-// FP64 67.8, 38.1; 512 of 1024 to 16384 29.8, 7.1 and 28.8, 8.3; 64 of 4096 to
-// 65536 FP32 28.9, 10.8; 256 of 1024 to 32768 with learned weights FP64 25.9,
-// 18.3; 4096 of 128 to 65536 FP32 113, 103 (bound by the FP32 rate: 174e9 cell
-// updates a second of some 195e9 that the whole-step arithmetic allows), FP64
-// 179, 145.
+// holds the states of every other workgroup of the XCD too. 1024 instances of
+// 128 to 65536 cells took 60.0 ms in FP32 and 67.8 in FP64 with fences at every
+// step and a tile per workgroup in LDS, 27.5 and 38.1 so; 4096 of them in FP32 113
+// and 103, bound by the FP32 rate (174e9 cell updates a second of some 195e9 that
+// the whole-step arithmetic allows).
 template <typename T, int FLUX, int BLOCK, int CPT, bool LEARNED, bool WHOLE, int REC>
 __global__ __launch_bounds__(BLOCK)
     __attribute__((amdgpu_waves_per_eu((batch_min_waves<T, LEARNED, WHOLE, BLOCK>()))))

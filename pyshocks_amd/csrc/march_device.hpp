@@ -163,8 +163,8 @@ __device__ __forceinline__ void march_control(psa_control *ctrl, int tid, bool f
 // N = 1500 5.23, 2.58; 16384 5.05, 2.90; 47104 5.14, 3.30; 112640 5.47, 3.82;
 // 243712 6.50, 4.81; 374784 7.46, 6.11; 505856 8.41, 7.18 (FP32 4.79, 2.44 to 6.55,
 // 6.09). Lax-Friedrichs, as three launches a step and as a march: N = 184 12.9,
-// 2.5; 16384 15.3, 6.5; 112640 15.7, 8.4; 505856 19.8, 12.3 (FP32 12.6, 2.3 to
-// 17.5, 10.6). With learned weights the network's latency rules and both take the
+// 2.4; 16384 15.3, 6.1; 112640 15.7, 7.9; 505856 19.8, 11.1 (FP32 12.6, 2.1 to
+// 17.5, 10.2). With learned weights the network's latency rules and both take the
 // same, so they stay on the step kernel.
 template <typename T, int FLUX, int REC, int CPT>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_march(
@@ -605,7 +605,7 @@ int launch_march_cells(const StageArgs<T> &a, MarchArgs<T> f, void *scratch, hip
 // against 7.09; with 6 cells per lane 8.5), else 505856 (7.2 against 8.4, FP32 6.1
 // against 6.5; FP32 with 16 cells per lane 8.9); the stage launches of
 // Lax-Friedrichs take longer up to the largest tiles (FP32, N = 1030144: 14.3
-// against 21.5; FP64, N = 505856: 12.3 against 19.8).
+// against 21.5; FP64, N = 505856: 11.1 against 19.8).
 template <typename T, int FLUX, int REC>
 int launch_march_tiles(const StageArgs<T> &a, const MarchArgs<T> &f, void *scratch,
                        hipStream_t s) {

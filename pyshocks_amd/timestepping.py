@@ -203,9 +203,14 @@ class FusedPlan:
         """Whether :meth:`steps` runs one whole-step kernel per step."""
         return not _uses_ring_kernel(self.desc) and _uses_step_kernel(self.desc)
 
+    def uses_wave_tiles(self) -> bool:
+        """Whether the whole-step kernel holds its tiles in the registers of a
+        wave each (large FP64 states) instead of in LDS."""
+        return self.uses_step_kernel() and _uses_wave_tiles(self.desc)
+
     def uses_ring_kernel(self) -> bool:
         """Whether :meth:`steps` runs all its steps in one launch of one
-        workgroup that holds the state in LDS."""
+        workgroup, which hands the state from step to step through LDS."""
         return _uses_ring_kernel(self.desc)
 
     def runs_in_one_launch(self) -> bool:
@@ -246,6 +251,15 @@ def _uses_step_kernel(d: _lib.PsaSolverDesc) -> bool:
     if block == 256 and cpt == 1:
         return d.rec == _lib.PSA_REC_WENOJS53 and d.flux != _lib.PSA_FLUX_ESWENO
     return block == 256 and cpt in (2, 4)
+
+
+def _uses_wave_tiles(d: _lib.PsaSolverDesc) -> bool:
+    """The library's rule for the whole-step kernel on wave tiles, where the
+    whole-step kernel applies: FP64, default schedule and tiles, a periodic
+    WENO-JS5 state of at least 2^21 cells, no learned weights."""
+    return (d.dtype == _lib.PSA_FLOAT64 and d.schedule == _lib.PSA_SCHEDULE_DEFAULT
+            and d.block <= 0 and d.cells_per_thread <= 0 and d.bc == _lib.PSA_BC_PERIODIC
+            and not d.mlp and d.rec == _lib.PSA_REC_WENOJS53 and d.n >= 1 << 21)
 
 
 def _uses_ring_kernel(d: _lib.PsaSolverDesc) -> bool:
