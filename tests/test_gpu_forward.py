@@ -17,6 +17,15 @@ RTOL64 = 1.0e-12
 RTOL32 = 1.0e-5
 
 
+@pytest.fixture(autouse=True)
+def default_tiles(monkeypatch) -> None:
+    """Plans with the library's own tiles, whatever sizes another test has tuned
+    (tuned tiles take other kernels)."""
+    from pyshocks_amd import autotune
+
+    monkeypatch.setattr(autotune, "_STAGE_CACHE", {})
+
+
 @pytest.fixture(scope="module")
 def torch_mod():
     import torch
