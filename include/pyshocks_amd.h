@@ -379,8 +379,8 @@ typedef struct psa_solver_desc {
  *   steps); every workgroup decides the step from the control block, loads
  *   its tile of u^n with a 12-cell margin on each side, runs the three
  *   stages in LDS (recomputing the margin cells of the first two; under DEFAULT
- *   large FP64 states in the registers of a wave per tile) and writes u^(n+1) (2 words per cell and step; any reconstruction, WENO-JS or
- *   learned weights, no velocity array, no Rusanov nu, not Lax-Friedrichs
+ *   large FP64 states in the registers of a wave per tile) and writes u^(n+1)
+ *   (2 words per cell and step; any reconstruction, WENO-JS or learned weights, no velocity array, no Rusanov nu, not Lax-Friedrichs
  *   (its stages need the global max|u| of the previous stage), a control
  *   block, tiles 256 x 4 or 256 x 2). Steps ping-pong between u_out and the
  *   stage buffers.

@@ -105,7 +105,9 @@ __device__ __forceinline__ void weno_cell_weights(T e0, T e1, T e2, T ie[3], T w
   }
   if (__builtin_expect(!fast, std::is_same<T, float>::value)) {
     using C = Weno5Coeffs<T>;
-    const T q0 = e0 * e0, q1 = e1 * e1, q2 = e2 * e2;
+    // (of eps + beta_k, a quarter: the squares' range)
+    const T f0 = T(0.25) * e0, f1 = T(0.25) * e1, f2 = T(0.25) * e2;
+    const T q0 = f0 * f0, q1 = f1 * f1, q2 = f2 * f2;
     const T a0 = C::d0 / q0, a1 = C::d1 / q1, a2 = C::d2 / q2;
     const T l0 = C::d2 / q0, l2 = C::d0 / q2;
     const T aR = (a0 + a1) + a2, aL = (l2 + a1) + l0;
@@ -739,8 +741,8 @@ constexpr int step_vjp_out(int nsub) { return kVjpBlock - 18 * nsub; }
 // arithmetic as k_stage_vjp, and the same bits whatever nsub.
 //
 // One step per launch is mostly launch, load and drain at the size of a single
-// gradient (N = 16384: 6.3 us a step, 3.1 of them the three stages), on a device that is nearly idle;
-// several share that cost, and the next step's states are loaded while this
+// gradient (N = 16384: 6.3 us a step, 3.1 of them the three stages), on a device
+// that is nearly idle; several share that cost, and the next step's states are loaded while this
 // one computes.
 // MANY: more than one step (the registers of the states in flight, 90 instead
 // of 66, would cost a batch a workgroup per CU).
@@ -1044,9 +1046,10 @@ int launch_vjp(const psa_solver_desc *d, int rstage, const void *state,
 }
 
 // Reverse steps that a launch best takes. Measured (FP64, Rusanov; us a step
-// with 1 step per launch and with the chosen number): one instance of 256 cells
-// 5.33 -> 3.41, of 16384 6.31 -> 3.41, of 65536 7.19 -> 4.48; 16 instances of
-// 16384 11.6 -> 9.5.
+// with 1 step per launch and with the chosen number, before the six operations
+// that keep the weights' gradients exact beside a jump, 2 to 3% more since): one
+// instance of 256 cells 5.33 -> 3.41, of 16384 6.31 -> 3.41, of 65536 7.19 -> 4.48;
+// 16 instances of 16384 11.6 -> 9.5.
 int reverse_steps_per_launch(const psa_solver_desc *d, long long batch) {
   return best_steps(StepCost{3.3, 2.0, 1.0}, kVjpMostSteps, [&](int k) {
     const int nout = step_vjp_out(k);

@@ -132,6 +132,34 @@ def test_operator_vjp_beside_a_jump(torch_mod, monkeypatch, velocity: float,
     assert np.abs(got[g:-g] - ref).max() <= 40 * 2.0**-53 * np.abs(ref).max()
 
 
+def test_operator_vjp_float32_range(torch_mod) -> None:
+    """FP32 gradients of large states: (eps + beta)^2 stays in range up to
+    differences of 1.5e9 from cell to cell (eps + beta carried four times as large
+    and squared would leave it at half of that). Against FP64, a dozen FP32
+    divisions and sums: 1e-5."""
+    torch = torch_mod
+    from pyshocks_amd import advection, make_uniform_cell_grid
+    from pyshocks_amd.adjoint import operator_vjp
+    from pyshocks_amd.reconstruction import WENOJS53
+    from pyshocks_amd.scalar import PeriodicBoundary
+    from pyshocks_amd.timestepping import BoundOperator
+
+    n = 40
+    rng = np.random.default_rng(5)
+    u = 0.6e9 * np.where(np.arange(n + 6) % 2 == 0, 1.0, -1.0) * rng.uniform(0.9, 1.0, n + 6)
+    u, mu = u.astype(np.float32), rng.standard_normal(n + 6).astype(np.float32)
+    got = []
+    for dtype in (torch.float32, torch.float64):
+        grid = make_uniform_cell_grid(0.0, 1.0, n, nghosts=3, dtype=dtype)
+        vel = torch.ones(n + 6, dtype=dtype, device="cuda")
+        src = BoundOperator(advection.Godunov(rec=WENOJS53(eps=1e-6), velocity=vel), grid,
+                            PeriodicBoundary())
+        got.append(_host(operator_vjp(src, torch.tensor(u, device="cuda").to(dtype),
+                                      torch.tensor(mu, device="cuda").to(dtype))))
+    assert np.isfinite(got[0]).all()
+    assert _rel(got[0], got[1]) < 1e-5
+
+
 @pytest.mark.parametrize("kind", KINDS_LF)
 @pytest.mark.parametrize("n", [40, 600])
 def test_step_vjp_vs_complex_step(torch_mod, kind: str, n: int) -> None:
